@@ -1,6 +1,7 @@
 """jaxpr -> HIP C++ emission for gfx950 (one program instance per lane)."""
 
 from palladium_amd.emit import rules as _rules  # noqa: F401  (registers RULES)
+from palladium_amd.emit import spread as _spread  # noqa: F401  (and the spread accesses')
 from palladium_amd.emit.core import (
     RULES,
     Cursor,

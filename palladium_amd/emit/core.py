@@ -443,7 +443,32 @@ class LaunchGeometry:
 
 
 def launch_geometry(spec: KernelSpec, block: int | None = None, lanes: int | None = None) -> LaunchGeometry:
-    from palladium_amd.emit.lanes import lanes_of, workgroup_for
+    return _geometry(spec, block, _UNPLANNED if lanes is None else lanes)
+
+
+_UNPLANNED: Any = object()
+
+
+def plan_of(spec: KernelSpec) -> Any:
+    """How the kernel's blocks are put on lanes: a `spread.SpreadPlan`, a
+    `lanes.LanePlan`, or None (one lane per instance). A function of the
+    traced kernel alone, so that every caller launches what was emitted."""
+    from palladium_amd.emit.lanes import lane_transform
+    from palladium_amd.emit.spread import own_rules, spread_transform
+
+    lanes = lane_transform(spec)
+    if not own_rules():
+        return lanes
+    memo = vars(spec)
+    if "_spread_plan" not in memo:
+        memo["_spread_plan"] = spread_transform(spec, lanes)
+    return memo["_spread_plan"] or lanes
+
+
+def _geometry(spec: KernelSpec, block: int | None, plan: Any) -> LaunchGeometry:
+    """`plan`: what `plan_of` returned, or a lane count."""
+    from palladium_amd.emit.lanes import workgroup_for
+    from palladium_amd.emit.spread import SpreadPlan
 
     n = spec.num_programs
     b = int(block) if block else DEFAULT_BLOCK
@@ -451,8 +476,12 @@ def launch_geometry(spec: KernelSpec, block: int | None = None, lanes: int | Non
         raise EmitError(f"block size {b} must be a positive multiple of 64 and at most 1024")
     if n <= 0:
         raise EmitError(f"grid {spec.grid} has no program instances")
-    lanes = lanes if lanes is not None else lanes_of(spec)
-    if lanes > 1:
+    if plan is _UNPLANNED:
+        plan = plan_of(spec)
+    lanes = plan if isinstance(plan, int) else (plan.lanes if plan is not None else 1)
+    if isinstance(plan, SpreadPlan):
+        b = plan.workgroup(block, DEFAULT_BLOCK)
+    elif lanes > 1:
         b = workgroup_for(lanes, block)
     else:
         from palladium_amd.emit.compact import WORKGROUP, plan_for
@@ -502,14 +531,17 @@ def emit_hip(spec: KernelSpec, kernel_name: str | None = None, block: int | None
     UnsupportedPrimitiveError
         A primitive with no registered rule.
     """
-    from palladium_amd.emit.prelude import PRELUDE
+    from palladium_amd.emit.prelude import PRELUDE, SPREAD_PRELUDE
 
-    from palladium_amd.emit.lanes import lane_transform
+    from palladium_amd.emit.spread import SpreadPlan, spread_jaxpr, spread_prologue
 
     name = kernel_name or spec.name
-    plan = lane_transform(spec)
-    lanes = plan.lanes if plan else 1
-    geo = launch_geometry(spec, block, lanes)
+    plan = plan_of(spec)
+    spread = plan if isinstance(plan, SpreadPlan) else None
+    if spread is not None:
+        plan = None
+    lanes = (spread or plan).lanes if spread or plan else 1
+    geo = _geometry(spec, block, spread or plan)
     operands = list(spec.inputs) + list(spec.outputs)
     n_in = len(spec.inputs)
     if len(spec.jaxpr.invars) != len(operands):
@@ -578,6 +610,8 @@ def emit_hip(spec: KernelSpec, kernel_name: str | None = None, block: int | None
     if keeps_compaction(pruned):
         body = pruned
 
+    if spread is not None:
+        body = spread_jaxpr(spec, spread, body)
     cplan = plan_for(spec, body, lanes, block)
     if (cplan is not None) != compacting:
         raise EmitError("internal: while-loop compaction disagrees with the launch geometry")
@@ -600,6 +634,8 @@ def emit_hip(spec: KernelSpec, kernel_name: str | None = None, block: int | None
     if lanes > 1:
         cursor.emit(f"const unsigned int _inst = _flat / {lanes}u;")
         cursor.emit(f"const int _lane = (int)(_flat % {lanes}u);")
+    if spread is not None:
+        spread_prologue(env, cursor, spread, geo.block)
     env.lanes = lanes  # type: ignore[attr-defined]
     env.math_mode = math_mode  # type: ignore[attr-defined]
     env.grid = tuple(spec.grid)  # type: ignore[attr-defined]
@@ -662,6 +698,7 @@ def emit_hip(spec: KernelSpec, kernel_name: str | None = None, block: int | None
         [
             f"// palladium_amd kernel {name}: grid={grid} block={geo.block} blocks={geo.blocks} lanes={lanes}",
             PRELUDE,
+            *([SPREAD_PRELUDE] if spread is not None and spread.reduces else []),
             head,
             *cursor.lines,
             "}",

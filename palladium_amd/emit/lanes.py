@@ -405,7 +405,15 @@ class _Pass:
 
 def lane_transform(spec: KernelSpec) -> LanePlan | None:
     """Per-lane rewrite of `spec.jaxpr`, or None when the kernel is not in
-    lane-separable form."""
+    lane-separable form. Found once per spec (bounds check, emission and
+    launch geometry all ask; a spec and its jaxpr are never changed)."""
+    memo = vars(spec)
+    if "_lane_plan" not in memo:
+        memo["_lane_plan"] = _lane_transform(spec)
+    return memo["_lane_plan"]
+
+
+def _lane_transform(spec: KernelSpec) -> LanePlan | None:
     found = _lane_count(spec)
     if found is None:
         return None

@@ -949,7 +949,7 @@ _PURE = frozenset((
     "shift_right_arithmetic shift_left clamp select_n integer_pow convert_element_type "
     "bitcast_convert_type fma pow_log pow_with_log get broadcast_in_dim reshape squeeze expand_dims "
     "transpose program_id num_programs random_wrap random_unwrap random_fold_in random_bits "
-    "threefry2x32 iota lane_index"
+    "threefry2x32 iota lane_index spread_index spread_get"
 ).split())
 
 

@@ -549,3 +549,37 @@ __device__ __forceinline__ float ph_pow(float x, float y) {
 __device__ __forceinline__ float ph_pow(float x, float y) { return powf(x, y); }
 #endif
 """
+
+# Only in kernels whose reductions run over a team of lanes (emit/spread.py).
+SPREAD_PRELUDE = r"""
+/* The value of the lane that DPP control CTRL pairs this one with: within
+   quads (quad_perm), between the quads of eight lanes (row_half_mirror) and
+   between the halves of sixteen (row_mirror). Lanes of one team are active
+   together, so no pair reads an inactive lane. */
+template <int CTRL, typename T> __device__ __forceinline__ T ph_dpp(T x) {
+    return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true));
+}
+/* Both halves of 32 (64) lanes in every lane: a the lower half's value, b
+   the upper half's. (Through scalars: this clang's __builtin_bit_cast of a
+   vector's element reads element 0.) */
+template <typename T> __device__ __forceinline__ void ph_swap16(T x, T& a, T& b) {
+    unsigned int v = __builtin_bit_cast(unsigned int, x);
+    auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    unsigned int r0 = r[0], r1 = r[1];
+    a = __builtin_bit_cast(T, r0);
+    b = __builtin_bit_cast(T, r1);
+}
+template <typename T> __device__ __forceinline__ void ph_swap32(T x, T& a, T& b) {
+    unsigned int v = __builtin_bit_cast(unsigned int, x);
+    auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    unsigned int r0 = r[0], r1 = r[1];
+    a = __builtin_bit_cast(T, r0);
+    b = __builtin_bit_cast(T, r1);
+}
+/* LDS writes of a wavefront before its later reads: its LDS operations run
+   in order, so only the compiler has to keep them so. */
+__device__ __forceinline__ void ph_wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+"""

@@ -1,0 +1,174 @@
+"""Kernels whose blocks are spread over teams of lanes (emit/spread.py),
+shared by the CPU and GPU tests: name -> (call factory, inputs). Sizes sit
+at the edges of the layout: one lane's chunk, a wavefront's, a ragged last
+chunk, the widest team, more than one run of slots."""
+
+import numpy as np
+
+import palladium_amd as pa
+from palladium_amd import dtypes
+from palladium_amd.frontend import jnp, lax, pl
+
+F = np.float32
+_DT = {"f32": np.dtype(np.float32), "f16": np.dtype(np.float16), "bf16": np.dtype(dtypes.bfloat16),
+       "i32": np.dtype(np.int32), "u32": np.dtype(np.uint32), "bool": np.dtype(np.bool_)}
+
+
+def _data(rng, shape, dt):
+    if dt in ("f32", "f16"):
+        return rng.standard_normal(shape).astype(_DT[dt])
+    if dt == "bf16":
+        return dtypes.from_float(rng.standard_normal(shape).astype(F))
+    if dt == "bool":
+        return rng.integers(0, 2, shape).astype(np.bool_)
+    return rng.integers(0, 100, shape).astype(_DT[dt])
+
+
+def flat(b, dt="f32", grid=5):
+    """Element by element over blocks of b."""
+    def kernel(x_ref, y_ref, o_ref):
+        x, y = x_ref[...], y_ref[...]
+        if dt == "bool":
+            o_ref[...] = jnp.logical_xor(x, y)
+        elif dt in ("i32", "u32"):
+            o_ref[...] = x * y + 3
+        else:
+            z = x * y + 0.25 * x
+            o_ref[...] = jnp.where(z > 0, z * 3.0, jnp.abs(y) - 0.5)
+
+    def make(rng, **kw):
+        s = pl.BlockSpec((b,), lambda i: (i,))
+        call = pa.hip_call(kernel, grid=(grid,), in_specs=[s, s], out_specs=s,
+                           out_shape=pl.ShapeDtypeStruct((grid * b,), _DT[dt]), **kw)
+        return call, (_data(rng, grid * b, dt), _data(rng, grid * b, dt))
+
+    return make
+
+
+def flat2d(m, w, grid=3):
+    """A whole block of rows, element by element, through two refs of other ranks."""
+    def kernel(x_ref, o_ref):
+        o_ref[...] = x_ref[...] * 2.0 + 1.0
+
+    def make(rng, **kw):
+        s = pl.BlockSpec((m, w), lambda i: (i, 0))
+        call = pa.hip_call(kernel, grid=(grid,), in_specs=[s], out_specs=s,
+                           out_shape=pl.ShapeDtypeStruct((grid * m, w), F), **kw)
+        return call, (_data(rng, (grid * m, w), "f32"),)
+
+    return make
+
+
+def rows(m, w, dt="f32", grid=3):
+    """Row maximum and sum, a row of biases, a value per row, both indices."""
+    fl = dt in ("f32", "f16", "bf16")
+
+    def kernel(x_ref, bias_ref, scale_ref, o_ref, top_ref, n_ref):
+        x = x_ref[...]
+        z = x + bias_ref[...]
+        top = jnp.max(z, axis=-1, keepdims=True)
+        low = jnp.min(z, axis=-1, keepdims=True)
+        i = lax.broadcasted_iota(jnp.int32, (m, w), 0)
+        j = lax.broadcasted_iota(jnp.int32, (m, w), 1)
+        total = jnp.sum(z, axis=-1, keepdims=True)
+        if fl:
+            o_ref[...] = (z - top) * 0.5 + total * 0.125 + scale_ref[...]
+        else:
+            o_ref[...] = (z - top) * 3 + total + scale_ref[...]
+        top_ref[...] = top - low
+        n_ref[...] = jnp.sum(jnp.where(z > low, i * w + j, -1), axis=-1)
+
+    def make(rng, **kw):
+        s = pl.BlockSpec((m, w), lambda i: (i, 0))
+        col = pl.BlockSpec((m, 1), lambda i: (i, 0))
+        call = pa.hip_call(kernel, grid=(grid,),
+                           in_specs=[s, pl.BlockSpec((w,), lambda i: (0,)), col],
+                           out_specs=(s, col, pl.BlockSpec((m,), lambda i: (i,))),
+                           out_shape=(pl.ShapeDtypeStruct((grid * m, w), _DT[dt]),
+                                      pl.ShapeDtypeStruct((grid * m, 1), _DT[dt]),
+                                      pl.ShapeDtypeStruct((grid * m,), np.int32)), **kw)
+        return call, (_data(rng, (grid * m, w), dt), _data(rng, (w,), dt), _data(rng, (grid * m, 1), dt))
+
+    return make
+
+
+def loops(b, grid=4):
+    """A loop whose carry starts the same everywhere, a loop until every
+    element is done, a switch on a reduction, any and all."""
+    def kernel(x_ref, o_ref, k_ref, f_ref):
+        x = x_ref[...]
+        y = lax.fori_loop(0, 7, lambda i, c: c * 0.5 + x * (i + 1), jnp.zeros((b,), jnp.float32))
+
+        def body(c):
+            v, n = c
+            return jnp.where(v > 1.0, v * 0.5, v), n + 1
+
+        v, n = lax.while_loop(lambda c: jnp.any(c[0] > 1.0), body, (jnp.abs(y) * 8.0, jnp.int32(0)))
+        t = jnp.max(x)
+        v = lax.cond(t > 2.0, lambda a: a - t, lambda a: a + 1.0, v)
+        o_ref[...] = v
+        k_ref[0] = n
+        f_ref[0] = jnp.all(v < 2.0)
+
+    def make(rng, **kw):
+        s = pl.BlockSpec((b,), lambda i: (i,))
+        one = pl.BlockSpec((1,), lambda i: (i,))
+        call = pa.hip_call(kernel, grid=(grid,), in_specs=[s], out_specs=(s, one, one),
+                           out_shape=(pl.ShapeDtypeStruct((grid * b,), F), pl.ShapeDtypeStruct((grid,), np.int32),
+                                      pl.ShapeDtypeStruct((grid,), np.bool_)), **kw)
+        return call, (_data(rng, grid * b, "f32"),)
+
+    return make
+
+
+def indexed(m, w, grid=3):
+    """Rows and columns of a block one by one: a column per row's first
+    lane, a row for all rows, single elements of a parameter array."""
+    def kernel(x_ref, p_ref, o_ref, c_ref, r_ref):
+        x = x_ref[...]
+        a, b = p_ref[0], p_ref[2]
+        o_ref[...] = x * a + b
+        c_ref[:, 1] = x_ref[:, 0] * 2.0
+        c_ref[:, 0] = jnp.sum(x, axis=1)
+        r_ref[0, :] = x_ref[1, :] + b
+
+    def make(rng, **kw):
+        s = pl.BlockSpec((m, w), lambda i: (i, 0))
+        call = pa.hip_call(kernel, grid=(grid,), in_specs=[s, pl.BlockSpec((3,), lambda i: (0,))],
+                           out_specs=(s, pl.BlockSpec((m, 2), lambda i: (i, 0)), pl.BlockSpec((1, w), lambda i: (i, 0))),
+                           out_shape=(pl.ShapeDtypeStruct((grid * m, w), F), pl.ShapeDtypeStruct((grid * m, 2), F),
+                                      pl.ShapeDtypeStruct((grid, w), F)), **kw)
+        return call, (_data(rng, (grid * m, w), "f32"), _data(rng, (3,), "f32"))
+
+    return make
+
+
+def single(n):
+    """One instance, looping over a whole array."""
+    def kernel(y_ref, r_ref, o_ref):
+        r = r_ref[...]
+        o_ref[...] = lax.fori_loop(0, 20, lambda _, y: y + 0.01 * r * y * (1.0 - y), y_ref[...])
+
+    def make(rng, **kw):
+        call = pa.hip_call(kernel, out_shape=pl.ShapeDtypeStruct((n,), F), **kw)
+        return call, (_data(rng, n, "f32"), _data(rng, n, "f32"))
+
+    return make
+
+
+CASES = {
+    **{f"flat_{b}_{dt}": flat(b, dt) for b, dt in
+       ((32, "f32"), (33, "f32"), (100, "f16"), (250, "bf16"), (1000, "u32"), (1025, "f32"), (1250, "bf16"),
+        (4096, "i32"), (5001, "f32"), (300, "bool"), (2048, "f16"))},
+    "flat_16_f32": flat(16, "f32"),
+    "flat_wide_1024_f16": flat(1024, "f16", grid=2000),
+    "flat_wide_f32": flat(1000, "f32", grid=1200),
+    "flat_wide_bf16": flat(1000, "bf16", grid=2400),
+    **{f"flat2d_{m}x{w}": flat2d(m, w) for m, w in ((3, 40), (8, 128), (7, 333), (1, 50))},
+    **{f"rows_{m}x{w}_{dt}": rows(m, w, dt) for m, w, dt in
+       ((1, 37, "f32"), (1, 64, "i32"), (1, 1000, "f32"), (1, 1025, "bf16"), (1, 3000, "f32"), (4, 17, "f32"),
+        (5, 33, "f16"), (8, 128, "f32"), (8, 100, "bf16"), (64, 40, "f32"), (64, 8, "f32"), (12, 4, "f32"), (300, 8, "f32"), (3, 700, "u32"), (33, 34, "f32"))},
+    **{f"loops_{b}": loops(b) for b in (48, 100, 777, 1500)},
+    **{f"indexed_{m}x{w}": indexed(m, w) for m, w in ((4, 24), (6, 130))},
+    **{f"single_{n}": single(n) for n in (65, 200, 1024, 3000)},
+}

@@ -1,0 +1,49 @@
+"""Blocks spread over teams of lanes on the GPU: SAFE and REPRODUCIBLE bit
+for bit against the interpreter (float sums in the traced order), FAST
+against float64."""
+
+import numpy as np
+import pytest
+
+from palladium_amd import dtypes
+from spread_cases import CASES
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(name, mode):
+    call, args = CASES[name](np.random.default_rng(7), math_mode=mode)
+    print(f"[spread] {name} {mode}", flush=True)
+    got, want = call(*args), call.interpret(*args)
+    return [got] if isinstance(got, np.ndarray) else got, [want] if isinstance(want, np.ndarray) else want
+
+
+@pytest.mark.parametrize("mode", ["safe", "reproducible"])
+@pytest.mark.parametrize("name", sorted(CASES))
+def test_bit_exact_against_the_interpreter(name, mode):
+    for g, w in zip(*_run(name, mode)):
+        if dtypes.is_bf16(g.dtype):
+            g, w = g.view(np.uint16), w.view(np.uint16)
+        np.testing.assert_array_equal(g, w)
+
+
+@pytest.mark.parametrize("name", sorted(n for n in CASES if not n.startswith("loops")))
+def test_fast_close_to_the_interpreter(name):
+    """FAST reassociates: a sum of n terms in another order moves by at most
+    n eps times the sum of magnitudes (n <= 5,001, standard normal data),
+    plus a few roundings of the element-wise part; narrow types round each
+    operation to their own eps."""
+    for g, w in zip(*_run(name, "fast")):
+        if dtypes.is_bf16(g.dtype):
+            g, w, eps = dtypes.to_float(g), dtypes.to_float(w), 2.0**-8
+        elif g.dtype.kind != "f":
+            np.testing.assert_array_equal(g, w)
+            continue
+        else:
+            eps = float(np.finfo(g.dtype).eps)
+        g, w = g.astype(np.float64), w.astype(np.float64)
+        # the interpreter's own ordered sum carries the larger part: n eps/2
+        # of a partial sum of about sqrt(n) in the narrow type
+        n = max(1, int(name.split("x")[1].split("_")[0])) if name.startswith("rows") else 64
+        scale = np.abs(w).max() + np.sqrt(n)
+        assert np.abs(g - w).max() <= 8 * eps * scale * np.sqrt(n)

@@ -1,0 +1,90 @@
+"""Blocks spread over teams of lanes, on the CPU: which kernels take the
+form, that its lanes cover every element once, and the forms it leaves to
+the other lowerings. (The results are compared on the GPU.)"""
+
+import numpy as np
+import pytest
+
+import palladium_amd as pa
+from palladium_amd.emit import emit_hip, launch_geometry
+from palladium_amd.emit.core import plan_of
+from palladium_amd.emit.spread import MAX_LANES, MAX_SLOTS, SpreadPlan
+from palladium_amd.frontend import jnp, pl
+from palladium_amd.trace import trace
+from spread_cases import CASES
+
+F = np.float32
+
+
+def _spec(name):
+    call, args = CASES[name](np.random.default_rng(1))
+    return trace(call._staged, *args)
+
+
+@pytest.mark.parametrize("name", sorted(CASES))
+def test_every_element_has_one_lane(name):
+    spec = _spec(name)
+    plan = plan_of(spec)
+    assert isinstance(plan, SpreadPlan)
+    assert 1 < plan.lanes <= MAX_LANES and plan.slots <= MAX_SLOTS and plan.slots % plan.vec == 0
+    seen = sorted(e for q in range(plan.chunks) for t in range(plan.team) for v in range(plan.vec)
+                  if (w := (q * plan.team + t) * plan.vec) < plan.width for e in [w + v])
+    assert seen == list(range(plan.width))
+    m, w = plan.block
+    assert plan.rows * plan.width == m * w
+    geo = launch_geometry(spec)
+    assert geo.lanes == plan.lanes and geo.block % 64 == 0
+    assert geo.blocks * geo.block >= spec.num_programs * plan.lanes
+    if plan.reduces:  # a team inside a wavefront, or a workgroup of its own
+        assert plan.team & (plan.team - 1) == 0
+        assert geo.block % plan.team == 0 and (plan.team <= 64 or geo.block == plan.team)
+
+
+@pytest.mark.parametrize("name", ["flat_1250_bf16", "rows_8x128_f32", "rows_1x3000_f32", "loops_777", "indexed_6x130"])
+@pytest.mark.parametrize("mode", ["safe", "relaxed", "fast", "reproducible"])
+def test_compiles_without_scratch(name, mode):
+    call, args = CASES[name](np.random.default_rng(1), math_mode=mode)
+    assert call.explain(*args).resources.scratch_bytes == 0
+
+
+def _row_call(kernel, m=4, w=64, out=None, **kw):
+    s = pl.BlockSpec((m, w), lambda i: (i, 0))
+    return pa.hip_call(kernel, grid=(3,), in_specs=[s], out_specs=s, out_shape=pl.ShapeDtypeStruct((3 * m, w), F), **kw)
+
+
+def _read_back(x_ref, o_ref):
+    o_ref[...] = x_ref[...]
+    o_ref[0, :] = o_ref[1, :] * 2.0
+
+
+def _across_rows(x_ref, o_ref):
+    o_ref[...] = x_ref[...] - jnp.sum(x_ref[...], axis=0, keepdims=True)
+
+
+def _transposed(x_ref, o_ref):
+    o_ref[...] = x_ref[...] + jnp.reshape(x_ref[...].T, (4, 64))
+
+
+def _part(x_ref, o_ref):
+    o_ref[0:2, :] = x_ref[0:2, :] * 2.0
+    o_ref[2:4, :] = x_ref[2:4, :]
+
+
+@pytest.mark.parametrize("kernel", [_read_back, _across_rows, _transposed, _part])
+def test_other_forms_keep_their_lowering(kernel):
+    """An output read where another lane wrote it, a reduction across rows,
+    a transpose, part of a block."""
+    spec = trace(_row_call(kernel)._staged, np.zeros((12, 64), F))
+    assert not isinstance(plan_of(spec), SpreadPlan)
+    emit_hip(spec, math_mode="fast")
+
+
+def test_small_blocks_and_plain_gridless_calls_keep_one_lane():
+    def double(x_ref, o_ref):
+        o_ref[...] = x_ref[...] * 2.0
+
+    s = pl.BlockSpec((15,), lambda i: (i,))
+    small = pa.hip_call(double, grid=(4,), in_specs=[s], out_specs=s, out_shape=pl.ShapeDtypeStruct((60,), F))
+    assert plan_of(trace(small._staged, np.zeros(60, F))) is None
+    whole = pa.hip_call(double, out_shape=pl.ShapeDtypeStruct((4096,), F))
+    assert plan_of(trace(whole._staged, np.zeros(4096, F))) is None
