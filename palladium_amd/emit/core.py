@@ -698,7 +698,7 @@ def emit_hip(spec: KernelSpec, kernel_name: str | None = None, block: int | None
         [
             f"// palladium_amd kernel {name}: grid={grid} block={geo.block} blocks={geo.blocks} lanes={lanes}",
             PRELUDE,
-            *([SPREAD_PRELUDE] if spread is not None and spread.reduces else []),
+            *([SPREAD_PRELUDE] if spread is not None and (spread.reduces or spread.tile) else []),
             head,
             *cursor.lines,
             "}",

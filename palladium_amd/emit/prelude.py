@@ -550,7 +550,8 @@ __device__ __forceinline__ float ph_pow(float x, float y) { return powf(x, y); }
 #endif
 """
 
-# Only in kernels whose reductions run over a team of lanes (emit/spread.py).
+# Only in kernels with reductions over a team of lanes, or with dots into
+# tiles (emit/spread.py).
 SPREAD_PRELUDE = r"""
 /* The value of the lane that DPP control CTRL pairs this one with: within
    quads (quad_perm), between the quads of eight lanes (row_half_mirror) and
@@ -576,6 +577,10 @@ template <typename T> __device__ __forceinline__ void ph_swap32(T x, T& a, T& b)
     a = __builtin_bit_cast(T, r0);
     b = __builtin_bit_cast(T, r1);
 }
+/* Operands and results of the matrix instructions. */
+typedef float ph_f32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 ph_bf16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 ph_f16x8 __attribute__((ext_vector_type(8)));
 /* LDS writes of a wavefront before its later reads: its LDS operations run
    in order, so only the compiler has to keep them so. */
 __device__ __forceinline__ void ph_wave_sync() {

@@ -143,6 +143,45 @@ def indexed(m, w, grid=3):
     return make
 
 
+def dense(m, k, n, dt="f32", grid=3, transposed=False):
+    """Rows times a matrix plus a bias and a value per row."""
+    def kernel(a_ref, w_ref, b_ref, s_ref, o_ref):
+        w = w_ref[...]
+        y = lax.dot_general(a_ref[...], w, (((1,), (1,)), ((), ()))) if transposed else jnp.dot(a_ref[...], w)
+        o_ref[...] = jnp.maximum(y + b_ref[...], 0.0) + s_ref[...]
+
+    def make(rng, **kw):
+        call = pa.hip_call(kernel, grid=(grid,),
+                           in_specs=[pl.BlockSpec((m, k), lambda i: (i, 0)),
+                                     pl.BlockSpec((n, k) if transposed else (k, n), lambda i: (0, 0)),
+                                     pl.BlockSpec((n,), lambda i: (0,)), pl.BlockSpec((m, 1), lambda i: (i, 0))],
+                           out_specs=pl.BlockSpec((m, n), lambda i: (i, 0)),
+                           out_shape=pl.ShapeDtypeStruct((grid * m, n), _DT[dt]), **kw)
+        return call, (_data(rng, (grid * m, k), dt), _data(rng, (n, k) if transposed else (k, n), dt), _data(rng, (n,), dt),
+                      _data(rng, (grid * m, 1), dt))
+
+    return make
+
+
+def two_dots(m, k, n, grid=3):
+    """Two products into one block, one of them with a matrix per instance, indices of both axes."""
+    def kernel(a_ref, w_ref, v_ref, o_ref):
+        y = jnp.dot(a_ref[...], w_ref[...]) - jnp.dot(a_ref[...], v_ref[...])
+        i = lax.broadcasted_iota(jnp.int32, (m, n), 0)
+        j = lax.broadcasted_iota(jnp.int32, (m, n), 1)
+        o_ref[...] = jnp.where(i > j, y, y * 0.5)
+
+    def make(rng, **kw):
+        call = pa.hip_call(kernel, grid=(grid,),
+                           in_specs=[pl.BlockSpec((m, k), lambda i: (i, 0)), pl.BlockSpec((k, n), lambda i: (0, 0)),
+                                     pl.BlockSpec((k, n), lambda i: (i, 0))],
+                           out_specs=pl.BlockSpec((m, n), lambda i: (i, 0)),
+                           out_shape=pl.ShapeDtypeStruct((grid * m, n), F), **kw)
+        return call, (_data(rng, (grid * m, k), "f32"), _data(rng, (k, n), "f32"), _data(rng, (grid * k, n), "f32"))
+
+    return make
+
+
 def single(n):
     """One instance, looping over a whole array."""
     def kernel(y_ref, r_ref, o_ref):
@@ -170,5 +209,12 @@ CASES = {
         (5, 33, "f16"), (8, 128, "f32"), (8, 100, "bf16"), (64, 40, "f32"), (64, 8, "f32"), (12, 4, "f32"), (300, 8, "f32"), (3, 700, "u32"), (33, 34, "f32"))},
     **{f"loops_{b}": loops(b) for b in (48, 100, 777, 1500)},
     **{f"indexed_{m}x{w}": indexed(m, w) for m, w in ((4, 24), (6, 130))},
+    **{f"dense_{m}x{k}x{n}_{dt}": dense(m, k, n, dt) for m, k, n, dt in
+       ((128, 64, 32, "f32"), (64, 21, 17, "f32"), (100, 33, 3, "f32"), (16, 16, 16, "f32"), (1024, 16, 48, "f32"),
+        (250, 40, 64, "bf16"), (64, 32, 30, "bf16"), (128, 96, 16, "f16"), (33, 7, 33, "f16"), (256, 128, 64, "f32"))},
+    "dense_64x24x20_transposed_f32": dense(64, 24, 20, "f32", transposed=True),
+    "dense_64x40x20_transposed_bf16": dense(64, 40, 20, "bf16", transposed=True),
+    "dense_wide_f32": dense(128, 24, 32, "f32", grid=600),
+    "two_dots_64x24x16": two_dots(64, 24, 16),
     **{f"single_{n}": single(n) for n in (65, 200, 1024, 3000)},
 }

@@ -44,6 +44,6 @@ def test_fast_close_to_the_interpreter(name):
         g, w = g.astype(np.float64), w.astype(np.float64)
         # the interpreter's own ordered sum carries the larger part: n eps/2
         # of a partial sum of about sqrt(n) in the narrow type
-        n = max(1, int(name.split("x")[1].split("_")[0])) if name.startswith("rows") else 64
+        n = max(1, int(name.split("x")[1].split("_")[0])) if name.startswith(("rows", "dense_1", "dense_2")) else 64
         scale = np.abs(w).max() + np.sqrt(n)
         assert np.abs(g - w).max() <= 8 * eps * scale * np.sqrt(n)

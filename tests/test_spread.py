@@ -27,6 +27,14 @@ def test_every_element_has_one_lane(name):
     plan = plan_of(spec)
     assert isinstance(plan, SpreadPlan)
     assert 1 < plan.lanes <= MAX_LANES and plan.slots <= MAX_SLOTS and plan.slots % plan.vec == 0
+    if plan.tile:
+        down, across = plan.tile
+        seen = [(lane // 64 * 16 * down + 16 * a + 4 * (lane % 64 // 16) + i, 16 * b + lane % 16)
+                for lane in range(plan.lanes) for a in range(down) for b in range(across) for i in range(4)]
+        assert len(seen) == plan.lanes * plan.slots
+        kept = [(r, c) for r, c in seen if r < plan.rows and c < plan.width]
+        assert sorted(kept) == [(r, c) for r in range(plan.rows) for c in range(plan.width)]
+        return
     seen = sorted(e for q in range(plan.chunks) for t in range(plan.team) for v in range(plan.vec)
                   if (w := (q * plan.team + t) * plan.vec) < plan.width for e in [w + v])
     assert seen == list(range(plan.width))
@@ -40,7 +48,8 @@ def test_every_element_has_one_lane(name):
         assert geo.block % plan.team == 0 and (plan.team <= 64 or geo.block == plan.team)
 
 
-@pytest.mark.parametrize("name", ["flat_1250_bf16", "rows_8x128_f32", "rows_1x3000_f32", "loops_777", "indexed_6x130"])
+@pytest.mark.parametrize("name", ["flat_1250_bf16", "rows_8x128_f32", "rows_1x3000_f32", "loops_777", "indexed_6x130",
+                                  "dense_128x64x32_f32", "dense_250x40x64_bf16", "two_dots_64x24x16"])
 @pytest.mark.parametrize("mode", ["safe", "relaxed", "fast", "reproducible"])
 def test_compiles_without_scratch(name, mode):
     call, args = CASES[name](np.random.default_rng(1), math_mode=mode)
