@@ -93,6 +93,13 @@ int ph_launch(ph_kernel *k, unsigned int grid_x, unsigned int grid_y,
 int ph_launch_ptrs(ph_kernel *k, unsigned int blocks, unsigned int block,
                    void *stream, void *const *ptrs, size_t n_ptrs, char **err);
 
+/* `count` launches in order on `stream`: launch i is kernels[i] over
+ * blocks[i] x block[i] lanes with the n_ptrs[i] pointers that follow those
+ * of the launches before it in `ptrs`. Stops at the first that fails. */
+int ph_launch_many(ph_kernel *const *kernels, const unsigned int *blocks,
+                   const unsigned int *block, const size_t *n_ptrs,
+                   void *const *ptrs, size_t count, void *stream, char **err);
+
 /* One synchronous dispatch of emitted source over host buffers: compile or
  * hit the cache, stage inputs host->device, launch
  * ceil(prod(grid) * lanes / block) workgroups of `block` threads (0 = 256),

@@ -263,11 +263,30 @@ int ph_launch(ph_kernel *k, unsigned int gx, unsigned int gy, unsigned int gz,
 int ph_launch_ptrs(ph_kernel *k, unsigned int blocks, unsigned int block,
                    void *stream, void *const *ptrs, size_t n_ptrs, char **err) {
   if (n_ptrs && !ptrs) return fail(err, PH_ERR_INVALID_ARGUMENT, "ph_launch_ptrs: null pointer array");
-  std::vector<void *> values(ptrs, ptrs + n_ptrs);
-  std::vector<void *> params(n_ptrs);
-  for (size_t i = 0; i < n_ptrs; ++i) params[i] = &values[i];
-  return ph_launch(k, blocks, 1, 1, block, 1, 1, 0, stream,
-                   n_ptrs ? params.data() : nullptr, err);
+  // The launch reads the pointers while it is called, so the caller's array
+  // itself serves as the values.
+  void *few[32];
+  std::vector<void *> many;
+  void **params = few;
+  if (n_ptrs > 32) {
+    many.resize(n_ptrs);
+    params = many.data();
+  }
+  for (size_t i = 0; i < n_ptrs; ++i) params[i] = const_cast<void **>(&ptrs[i]);
+  return ph_launch(k, blocks, 1, 1, block, 1, 1, 0, stream, n_ptrs ? params : nullptr, err);
+}
+
+int ph_launch_many(ph_kernel *const *kernels, const unsigned int *blocks,
+                   const unsigned int *block, const size_t *n_ptrs,
+                   void *const *ptrs, size_t count, void *stream, char **err) {
+  if (count && (!kernels || !blocks || !block || !n_ptrs))
+    return fail(err, PH_ERR_INVALID_ARGUMENT, "ph_launch_many: null argument");
+  for (size_t i = 0; i < count; ++i) {
+    int rc = ph_launch_ptrs(kernels[i], blocks[i], block[i], stream, ptrs, n_ptrs[i], err);
+    if (rc != PH_OK) return rc;
+    ptrs += n_ptrs[i];
+  }
+  return PH_OK;
 }
 
 namespace {

@@ -137,6 +137,12 @@ class BoundKernel:
     _ring_next: list[int] = dataclasses.field(default_factory=lambda: [0], compare=False, repr=False)
     _launch_lock: threading.Lock = dataclasses.field(default_factory=threading.Lock, compare=False, repr=False)
     _stream: list[rt.Stream] = dataclasses.field(default_factory=list, compare=False, repr=False)
+    _forms: tuple = dataclasses.field(default=(), compare=False, repr=False)
+
+    def __post_init__(self) -> None:
+        # (dtype, shape) of every operand, inputs then outputs
+        object.__setattr__(self, "_forms", tuple((np.dtype(i.dtype), tuple(i.array_shape))
+                                                 for i in (*self.spec.inputs, *self.spec.outputs)))
 
     @property
     def stream(self) -> rt.Stream:
@@ -242,18 +248,25 @@ class BoundKernel:
         Buffers, torch tensors on the GPU, or `__cuda_array_interface__`
         objects. No copies, no synchronisation; shapes and dtypes are
         checked against the spec."""
-        infos = list(self.spec.inputs) + list(self.spec.outputs)
-        if len(operands) != len(infos):
-            raise DispatchError(f"kernel takes {len(infos)} device operands (inputs then outputs), got {len(operands)}")
+        expected = self._forms
+        if len(operands) != len(expected):
+            raise DispatchError(
+                f"kernel takes {len(expected)} device operands (inputs then outputs), got {len(operands)}")
         ptrs = []
-        for i, (o, info) in enumerate(zip(operands, infos)):
+        for i, o in enumerate(operands):
+            dtype, shape = expected[i]
+            if getattr(o, "is_cuda", False) and o.shape == shape and o.is_contiguous() and rt.torch_dtype(o.dtype) == dtype:
+                # a torch tensor of the right form, without the Buffer around it
+                # (1.5 us each; a call of three operands 18 -> 7 us)
+                ptrs.append(o.data_ptr())
+                continue
             b = o if isinstance(o, rt.Buffer) else rt.Buffer.wrap(o)
-            if b.dtype != info.dtype:
+            if b.dtype != dtype:
                 raise DispatchError(
-                    f"operand {i}: dtype {_dtype_name(b.dtype)} does not match the traced {_dtype_name(info.dtype)}"
+                    f"operand {i}: dtype {_dtype_name(b.dtype)} does not match the traced {_dtype_name(dtype)}"
                 )
-            if b.shape != tuple(info.array_shape):
-                raise DispatchError(f"operand {i}: expected shape {info.array_shape}, got {b.shape}")
+            if b.shape != shape:
+                raise DispatchError(f"operand {i}: expected shape {shape}, got {b.shape}")
             ptrs.append(b.ptr)
         geo = self._geo()
         self.kernel.launch_ptrs(geo.blocks, geo.block, ptrs, stream if stream is not None else self.stream)

@@ -468,7 +468,8 @@ class RegisterGrayScott:
 
 def gray_scott_fused_run(fused: FusedGrayScott | RegisterGrayScott, u0: np.ndarray, v0: np.ndarray, steps: int, graph: bool = True):
     """`steps` Gray-Scott steps in passes of `fused.k`, ping-ponging two
-    buffer pairs, queued as one batch (one HIP graph when `graph`).
+    buffer pairs, queued as one batch, which runs once and so is submitted
+    launch by launch whatever `graph` says (`workloads.gray_scott_run`).
     Returns (u, v, device seconds)."""
     if u0.shape != (fused.n, fused.n) or v0.shape != u0.shape:
         raise ValueError(f"fields must be {fused.n}x{fused.n}")
@@ -483,11 +484,11 @@ def gray_scott_fused_run(fused: FusedGrayScott | RegisterGrayScott, u0: np.ndarr
     ]
     stream = rt.Stream()
     batch = rt.Batch(stream=stream)
-    src = 0
-    for kk in fused.launches(steps):
-        dst = 1 - src
-        batch.add(fused._kernels[kk], fused.blocks_for(kk), WORKGROUP, [b.ptr for b in bufs[src]] + [b.ptr for b in bufs[dst]])
-        src = dst
-    batch.commit(graph=graph)
+    ptrs = [[b.ptr for b in bufs[src]] + [b.ptr for b in bufs[1 - src]] for src in (0, 1)]
+    passes = fused.launches(steps)
+    for i, kk in enumerate(passes):
+        batch.add(fused._kernels[kk], fused.blocks_for(kk), WORKGROUP, ptrs[i % 2])
+    batch.commit()
     batch.wait()
-    return bufs[src][0].to_numpy(stream), bufs[src][1].to_numpy(stream), batch.gpu_time
+    u, v = bufs[len(passes) % 2]
+    return u.to_numpy(stream), v.to_numpy(stream), batch.gpu_time
