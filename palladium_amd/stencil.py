@@ -202,6 +202,27 @@ def register_geometry(n: int, k: int, rows: int, cols: int = 1) -> tuple[int, in
     return waves, -(-waves // (WORKGROUP // WAVE))
 
 
+DEFAULT_ROWS = 64
+SIMDS = 1024
+
+
+def strip_height(n: int, k: int, rows: int = DEFAULT_ROWS, group: int = 4) -> int:
+    """The strip height up to `rows` for a pass over n x n. A wave walks its
+    strip and 2K halo rows in groups; with c waves on a SIMD a row costs
+    about 0.17 + 0.13 c us (issue: one wave leaves gaps that others fill), so
+    the height taken is the one with the least (walked rows) (c + 1.3). Small
+    grids get short strips, since their waves would otherwise leave SIMDs
+    empty: a six-step pass takes 21.3 -> 5.8 us at 200 (64 rows -> 2), 22.0
+    -> 7.6 at 512 (6), 22.6 -> 12.0 at 1024 (12), 31.5 -> 25.5 at 2048 (16),
+    42.8 -> 41.8 at 3000 (48); at 4096 64 rows stay best (62.5 us, 64.7 with
+    48)."""
+    def cost(r: int) -> float:
+        walked = -(-(r + 2 * k) // group) * group
+        return walked * (-(-register_geometry(n, k, r)[1] * (WORKGROUP // WAVE) // SIMDS) + 1.3)
+
+    return min(range(min(2, rows), rows + 1, 2), key=cost)
+
+
 def register_source(n: int, k: int, rows: int, du: float, dv: float, f: float, fk: float, dt: float,
                     group: int = 8, cols: int = 1) -> str:
     """HIP source of a K-step Gray-Scott pass with no LDS: each wave owns a
@@ -435,7 +456,10 @@ def _consts(cfg: Any) -> tuple:
 @dataclasses.dataclass
 class RegisterGrayScott:
     """A compiled K-step register pass (`register_source`) and a one-step
-    pass of the same code for step counts K does not divide."""
+    pass of the same code for step counts K does not divide. `rows` other
+    than the default is the height of the strips as given; at the default it
+    is the tallest that `strip_height` may choose. Results do not depend on
+    it."""
 
     n: int
     k: int = 6
@@ -447,16 +471,19 @@ class RegisterGrayScott:
 
     def __post_init__(self) -> None:
         consts = _consts(self.cfg)
-        self._src = {kk: register_source(self.n, kk, self.rows, *consts, group=self.group, cols=self.cols)
-                     for kk in {self.k, 1}}
+        chosen = self.rows == DEFAULT_ROWS and self.cols == 1 and self.rows + 2 * self.k <= self.n
+        height = strip_height(self.n, self.k, self.rows, self.group) if chosen else self.rows
+        self._rows = {kk: height for kk in {self.k, 1}}
+        self._src = {kk: register_source(self.n, kk, r, *consts, group=self.group, cols=self.cols)
+                     for kk, r in self._rows.items()}
         self._kernels = {kk: rt.Kernel(src, "gray_scott_regs", self.math_mode) for kk, src in self._src.items()}
-        self._blocks = {kk: register_geometry(self.n, kk, self.rows, self.cols)[1] for kk in self._src}
+        self._blocks = {kk: register_geometry(self.n, kk, r, self.cols)[1] for kk, r in self._rows.items()}
 
     def blocks_for(self, k: int) -> int:
         return self._blocks[k]
 
     def describe(self) -> str:
-        return (f"register pass: {self.rows}x{WAVE * self.cols - 2 * self.k} strips, one wave each, "
+        return (f"register pass: {self._rows[self.k]}x{WAVE * self.cols - 2 * self.k} strips, one wave each, "
                 f"{self.cols} column(s) per lane, rows in groups of {self.group}")
 
     def source(self, k: int | None = None) -> str:
