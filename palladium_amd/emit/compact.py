@@ -109,6 +109,7 @@ _STORABLE = {"float32": 1, "int32": 1, "uint32": 1, "bool": 1, "float64": 2}
 @dataclasses.dataclass(frozen=True)
 class CompactPlan:
     index: int  # position of the loop among the top-level eqns
+    workgroup: int  # lanes that repack together
 
 
 def _jaxpr(j: Any) -> Any:
@@ -139,6 +140,20 @@ def enabled() -> bool:
     return os.environ.get("PALLADIUM_WHILE_COMPACTION", "1") != "0"
 
 
+def workgroup_for(instances: int) -> int:
+    """Lanes that repack together. Above 131,072 instances (two wavefronts on
+    each of the 1,024 SIMDs) whole 1,024-lane workgroups, whose four waves a
+    SIMD pack best. Below, a large workgroup crowds its waves onto one CU
+    while others stand empty: BS3 (REPRODUCIBLE, 2,646 attempts at most) in
+    1,024 / 512 / 256 lanes takes 1,155 / 883 / 782 us at 65,536 instances,
+    1,132 / 869 / 778 at 5,000, 1,158 / 888 / 907 at 131,072, but 1,163 /
+    1,237 / 1,277 at 200,000. Up to 4,096 instances the geometry is the
+    documented one, 1,024 lanes."""
+    if instances <= 4096 or instances > 131_072:
+        return WORKGROUP
+    return 256 if instances <= 65_536 else 512
+
+
 def plan_for(spec: Any, jaxpr: Any, lanes: int, block: int | None) -> CompactPlan | None:
     """The loop to compact, or None. Needs: one lane per instance, a 1-D
     grid, no explicit workgroup size other than 1,024, and exactly one
@@ -165,7 +180,7 @@ def plan_for(spec: Any, jaxpr: Any, lanes: int, block: int | None) -> CompactPla
     n_kept = sum(_nwords(v) for v in e.outvars if v in used)  # final carries read after the loop
     if (n_state + n_kept) * WORKGROUP * 4 > LDS_BUDGET:
         return None
-    return CompactPlan(whiles[0])
+    return CompactPlan(whiles[0], block or workgroup_for(spec.num_programs))
 
 
 def _nwords(v: Any) -> int:
@@ -225,12 +240,13 @@ def emit_compacting_while(env: Any, cursor: Any, eqn: Any, emit_jaxpr: Any, decl
     carries = declare_carries(env, cursor, eqn.invars[cn + bn:], eqn.outvars)
     state = consts + carries
     kept = [(k, c) for k, (c, ov) in enumerate(zip(carries, eqn.outvars)) if env.used(ov)]
-    nw = WORKGROUP // 64
+    workgroup = env.compact_workgroup
+    nw = workgroup // 64
     buf, res, cnt = cursor.fresh("_cbuf"), cursor.fresh("_cres"), cursor.fresh("_ccnt")
     n_rows, kept_vals = _rows(state), [c for _, c in kept]
-    cursor.emit(f"__shared__ unsigned int {buf}[{n_rows + 1}][{WORKGROUP}];")
+    cursor.emit(f"__shared__ unsigned int {buf}[{n_rows + 1}][{workgroup}];")
     if kept:
-        cursor.emit(f"__shared__ unsigned int {res}[{_rows(kept_vals)}][{WORKGROUP}];")
+        cursor.emit(f"__shared__ unsigned int {res}[{_rows(kept_vals)}][{workgroup}];")
     cursor.emit(f"__shared__ int {cnt}[{nw}];")
     slot, own = cursor.fresh("_slot"), cursor.fresh("_own")
     first = f"(_in ? (int)threadIdx.x : -1)" if getattr(env, "compact_in", None) else "(int)threadIdx.x"

@@ -484,10 +484,11 @@ def _geometry(spec: KernelSpec, block: int | None, plan: Any) -> LaunchGeometry:
     elif lanes > 1:
         b = workgroup_for(lanes, block)
     else:
-        from palladium_amd.emit.compact import WORKGROUP, plan_for
+        from palladium_amd.emit.compact import plan_for
 
-        if plan_for(spec, spec.jaxpr, lanes, block) is not None:
-            b = WORKGROUP  # a compacting while loop repacks 1,024-lane workgroups
+        cplan = plan_for(spec, spec.jaxpr, lanes, block)
+        if cplan is not None:
+            b = cplan.workgroup  # a compacting while loop repacks whole workgroups
     threads = n * lanes
     if threads >= 2**31:
         raise EmitError(f"grid {spec.grid} needs more than 2**31 lanes")
@@ -567,7 +568,7 @@ def emit_hip(spec: KernelSpec, kernel_name: str | None = None, block: int | None
     # adds or removes loop carries can move a loop across the LDS budget of
     # lane compaction, so each such rewrite is taken only if it leaves the
     # loop's compaction as the geometry has it.
-    compacting = plan is None and geo.block == 1024 and plan_for(spec, spec.jaxpr, lanes, block) is not None
+    compacting = plan is None and plan_for(spec, spec.jaxpr, lanes, block) is not None
 
     def keeps_compaction(candidate: Jaxpr) -> bool:
         return (plan_for(spec, candidate, lanes, block) is not None) == compacting
@@ -687,6 +688,7 @@ def emit_hip(spec: KernelSpec, kernel_name: str | None = None, block: int | None
         ref_vals.append(CVal(f"arg{k}", info.block_shape or (1,), ct, "global", k < n_in))
 
     env.compact = body.eqns[cplan.index] if cplan is not None else None  # type: ignore[attr-defined]
+    env.compact_workgroup = geo.block  # type: ignore[attr-defined]
     emit_jaxpr(env, cursor, body, ref_vals)
 
     head = (

@@ -452,6 +452,9 @@ def synchronize_stream(stream: Any) -> None:
 def device_pointer(obj: Any) -> int:
     if isinstance(obj, Buffer):
         return obj.ptr
+    if hasattr(obj, "data_ptr") and getattr(obj, "is_cuda", False) and obj.is_contiguous():
+        torch_dtype(obj.dtype)  # a type Buffer.wrap refuses is refused here too
+        return obj.data_ptr()
     return Buffer.wrap(obj).ptr
 
 
@@ -528,7 +531,7 @@ class Kernel:
                 holders.append(ctypes.c_int(a))
             else:
                 holders.append(ctypes.c_void_p(device_pointer(a)))
-        params = (ctypes.c_void_p * max(len(holders), 1))(*[ctypes.cast(ctypes.pointer(x), ctypes.c_void_p) for x in holders])
+        params = _pointer_array(len(holders) or 1)(*map(ctypes.addressof, holders))  # `holders` lives until the launch returns
         g = tuple(grid) + (1,) * (3 - len(grid))
         b = tuple(block) + (1,) * (3 - len(block))
         _call("ph_launch", ctypes.c_void_p(h), *[ctypes.c_uint(x) for x in g], *[ctypes.c_uint(x) for x in b],
