@@ -38,6 +38,9 @@ __all__ = ["BoundKernel", "PendingResult", "bind"]
 
 # Launches a BoundKernel keeps in flight before `launch` blocks.
 IN_FLIGHT = 4
+# Inputs that together take at most this many bytes go up as one copy from
+# pinned memory; past it the extra copy on the host costs more than it saves.
+PACK_LIMIT = 64 * 1024
 
 
 def _dump_hip(name: str, source: str) -> None:
@@ -131,7 +134,7 @@ class BoundKernel:
     # pinned host staging for the outputs) serves launches k, k + IN_FLIGHT,
     # ...; a launch waits only for the last launch that used its set, so
     # uploads, kernels and readbacks of successive calls overlap.
-    _ring: list[tuple[list[rt.Buffer], list[rt.Buffer], list[rt.PinnedBuffer]]] = dataclasses.field(
+    _ring: list[tuple] = dataclasses.field(
         default_factory=list, compare=False, repr=False)
     _ring_pending: list[PendingResult | None] = dataclasses.field(default_factory=list, compare=False, repr=False)
     _ring_next: list[int] = dataclasses.field(default_factory=lambda: [0], compare=False, repr=False)
@@ -191,25 +194,48 @@ class BoundKernel:
             k = self._ring_next[0]
             self._ring_next[0] = (k + 1) % IN_FLIGHT
             if len(self._ring) <= k:
-                outs = self._new_outputs()
-                self._ring.append(([rt.Buffer.empty(a.shape, a.dtype) for a in arrs], outs,
-                                   [rt.PinnedBuffer(b.nbytes) for b in outs]))
+                self._ring.append(self._new_set(arrs))
                 self._ring_pending.append(None)
             previous = self._ring_pending[k]
             if previous is not None:
                 previous._settle()  # its outputs leave the set's staging first
-            in_bufs, out_bufs, staging = self._ring[k]
+            in_bufs, out_bufs, staging, packed = self._ring[k]
             stream = self.stream
-            for buf, a in zip(in_bufs, arrs):
-                buf.copy_from(a, stream)
+            if packed is None:
+                for buf, a in zip(in_bufs, arrs):
+                    buf.copy_from(a, stream)
+            else:
+                pinned, whole, views = packed
+                for view, a in zip(views, arrs):
+                    view[...] = a
+                whole.copy_from_pinned(pinned, stream)
             geo = self._geo()
             self.kernel.launch_ptrs(geo.blocks, geo.block, [b.ptr for b in in_bufs] + [b.ptr for b in out_bufs], stream)
             for pin, buf in zip(staging, out_bufs):
                 pin.copy_from_device(buf, stream)
-            pending = PendingResult(rt.Event().record(stream), out_bufs, stream, host_inputs=tuple(arrs),
-                                    staged=list(staging))
+            pending = PendingResult(rt.Event().record(stream), out_bufs, stream,
+                                    host_inputs=tuple(arrs) if packed is None else packed, staged=list(staging))
             self._ring_pending[k] = pending
             return pending
+
+    def _new_set(self, arrs: list[np.ndarray]) -> tuple:
+        """One buffer set: inputs, outputs, the outputs' pinned staging, and
+        for inputs of up to PACK_LIMIT bytes together a pinned area that they
+        go up from as one copy (an upload of its own costs each about 5 us)."""
+        outs = self._new_outputs()
+        staging = [rt.PinnedBuffer(b.nbytes) for b in outs]
+        starts, end = [], 0
+        for a in arrs:
+            starts.append(end)
+            end += -(-a.nbytes // 256) * 256
+        if not arrs or end > PACK_LIMIT:
+            return [rt.Buffer.empty(a.shape, a.dtype) for a in arrs], outs, staging, None
+        whole = rt.Buffer.empty((end,), np.uint8)
+        pinned = rt.PinnedBuffer(end)
+        ins = [rt.Buffer(a.shape, a.dtype, ptr=whole.ptr + at, owner=whole) for a, at in zip(arrs, starts)]
+        area = pinned.view((end,), np.uint8)
+        views = [area[at:at + a.nbytes].view(a.dtype).reshape(a.shape) for a, at in zip(arrs, starts)]
+        return ins, outs, staging, (pinned, whole, views)
 
     def __call__(self, *arrays: np.ndarray) -> np.ndarray | tuple[np.ndarray, ...]:
         """Launch over the grid and return the outputs (NumPy)."""

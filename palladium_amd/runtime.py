@@ -394,6 +394,12 @@ class Buffer:
             if stream is None or src is not arr:
                 synchronize_stream(stream)
 
+    def copy_from_pinned(self, pinned: "PinnedBuffer", stream: Any = None) -> None:
+        """Enqueue pinned memory -> this buffer on `stream` (returns at once;
+        the memory stays as it is until the stream passes this point)."""
+        if self.nbytes:
+            _call("ph_memcpy_h2d", self.ptr, pinned.ptr, self.nbytes, _stream_value(stream))
+
     def to_numpy(self, stream: Any = None) -> np.ndarray:
         """Copy to a new host array after the work queued on `stream`."""
         out = np.empty(self.shape, self.dtype)
