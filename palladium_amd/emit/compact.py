@@ -5,9 +5,10 @@ its slowest lane finishes; on config 2 (Van der Pol, mu log-uniform) half
 the lane-attempts of a wavefront do no work. When a kernel's loop runs one
 program instance per lane with nothing lane-specific inside it, the
 instance is only its loop state: the carries and the loop's operands. Then
-the state of a live instance can move to another lane, and a 1,024-lane
-workgroup can repack its live instances into its lowest wavefronts every
-`EPOCH` iterations, so emptied wavefronts stop issuing:
+the state of a live instance can move to another lane, and a workgroup (256
+to 1,024 lanes, see `workgroup_for`) can repack its live instances into its
+lowest wavefronts every `EPOCH` iterations, so emptied wavefronts stop
+issuing:
 
     epoch:  run up to EPOCH predicated iterations (a wavefront leaves the
             epoch early once none of its lanes is live);
@@ -19,6 +20,20 @@ workgroup can repack its live instances into its lowest wavefronts every
             mbcnt) and lanes [0, live) read it back;
             stop when no lane of the workgroup is live.
     after:  every lane reloads its own instance's final carries.
+
+Two things bound such a kernel: the iterations issued, and the one instance
+with the most of them, whose wavefront is latency-bound (BS3: a SIMD with w
+waves takes 137 + 117 w ns for an iteration of each, a lone wave 290 ns, and
+2,646 iterations lie between start and end of the longest instance). In
+lockstep epochs a long instance runs at the pace of the four waves on its
+SIMD while they last, and alone afterwards. Where the loop's condition tells
+how far an instance is (a float carry that starts at a constant and stays
+below a bound), each epoch ends with an estimate of its remaining iterations,
+(bound - carry) / progress per iteration so far; a histogram of the estimates
+in LDS gives the line above which the longest 256 lie, these move to the
+first four wavefronts (one a SIMD) and get three epochs' iterations to the
+others' one. The estimate only places instances: a wrong one costs time and
+changes no result.
 
 Each instance runs exactly the operations it ran before, in the same
 order: results are bit-identical with and without compaction. Wavefront w
@@ -40,7 +55,7 @@ from typing import Any
 
 import numpy as np
 
-from palladium_amd.ir import KeyAval
+from palladium_amd.ir import KeyAval, Literal, Var
 
 WORKGROUP = 1024
 EPOCH = 64
@@ -145,9 +160,9 @@ def workgroup_for(instances: int) -> int:
     each of the 1,024 SIMDs) whole 1,024-lane workgroups, whose four waves a
     SIMD pack best. Below, a large workgroup crowds its waves onto one CU
     while others stand empty: BS3 (REPRODUCIBLE, 2,646 attempts at most) in
-    1,024 / 512 / 256 lanes takes 1,155 / 883 / 782 us at 65,536 instances,
-    1,132 / 869 / 778 at 5,000, 1,158 / 888 / 907 at 131,072, but 1,163 /
-    1,237 / 1,277 at 200,000. Up to 4,096 instances the geometry is the
+    1,024 / 512 / 256 lanes takes 1,155 / 883 / 782 us at 65,536 instances and
+    1,132 / 869 / 778 at 5,000; with `_ranking` 1,024 / 512 lanes take 882 /
+    803 us at 131,072 and 892 / 1,004 at 262,144. Up to 4,096 instances the geometry is the
     documented one, 1,024 lanes."""
     if instances <= 4096 or instances > 131_072:
         return WORKGROUP
@@ -218,8 +233,116 @@ def _load(arr: str, j: int, pos: str, c: Any) -> tuple[str, int]:
     return f"{e} = ({t})({w});", j + 1
 
 
+def _progress(eqn: Any, producers: dict) -> tuple[int, Any, float] | None:
+    """(carry, bound, start) when the loop runs while a float32 carry that
+    starts at a literal stays below a bound (an integrator's time, say); the
+    bound is a literal or one of the condition's operands."""
+    cn, bn = int(eqn.params["cond_nconsts"]), int(eqn.params["body_nconsts"])
+    cj = _jaxpr(eqn.params["cond_jaxpr"])
+    made = {ov: e for e in cj.eqns for ov in e.outvars}
+    todo, tests = [cj.outvars[0]], []
+    while todo:
+        v = todo.pop()
+        e = made.get(v) if isinstance(v, Var) else None
+        if e is None:
+            continue
+        if e.primitive.name == "and":
+            todo.extend(e.invars)
+        elif e.primitive.name in ("lt", "le"):
+            tests.append((e.invars[0], e.invars[1]))
+        elif e.primitive.name in ("gt", "ge"):
+            tests.append((e.invars[1], e.invars[0]))
+    carries = {v: k for k, v in enumerate(cj.invars[cn:])}
+    for low, high in tests:
+        if not isinstance(low, Var) or low not in carries or np.dtype(low.aval.dtype) != np.float32:
+            continue
+        if not isinstance(high, Literal) and high not in cj.invars[:cn]:
+            continue
+        start = eqn.invars[cn + bn + carries[low]]
+        while isinstance(start, Var):
+            e = producers.get(start)
+            start = e.invars[0] if e is not None and e.primitive.name == "broadcast_in_dim" else None
+        if isinstance(start, Literal):
+            return carries[low], high, float(start.val)
+    return None
+
+
 def _rows(vals: list) -> int:
     return sum(2 if c.ctype == "double" else 1 for c in vals)
+
+
+# Ranking by progress: bins of the estimate (eight an octave), waves that take
+# the instances with the most to do, and their epochs in those of the others.
+RANK_BINS = 256
+RANK_WAVES = 4
+RANK_TURNS = 3
+# Ranked only while the estimates' quartiles lie this many bins apart: with
+# trip counts within 10 % of each other two or one bins would rank as well, and
+# cost 10-60 % (563 -> 637 us, 77 -> 129).
+RANK_SPREAD = 3
+# The smallest body (equations) that is ranked. The counting costs 6-15 us a
+# kernel whatever the body holds: 135 -> 141 us with 18 equations, 201 -> 205
+# with 34, 526 -> 522 with 130 (1,000 trips each, 262,144 instances), while
+# trip counts spread over 100-3,000 gain from 18 equations on in SAFE
+# (261 -> 248, 557 -> 507, 952 -> 841 us with 18, 66, 130).
+RANK_OPS = 64
+
+
+def _ranking(env: Any, eqn: Any, workgroup: int, rows: int) -> tuple | None:
+    """`_progress(eqn)` where ranking pays, else None: above 65,536 instances,
+    where a workgroup puts more than one wave on a SIMD, and with room in LDS
+    for the counts. BS3, REPRODUCIBLE / SAFE: 1,162 -> 902 / 1,927 -> 1,550 us
+    at 262,144 instances, 883 -> 805 / 1,399 -> 1,228 at 131,072 (workgroups
+    of 512), 4,590 -> 3,565 / 7,620 -> 6,157 at 1,048,576; three epochs against
+    two, four and six: 926 / 990 / 1,032 / 1,180 us. FAST keeps its order: its
+    text is held as a snapshot (672 -> 533 us when it is ranked)."""
+    from palladium_amd.runtime import math_mode_ordinal
+
+    mode = getattr(env, "math_mode", None)
+    if mode is None or math_mode_ordinal(mode) == 2 or env.compact_instances <= 65_536:
+        return None
+    if rows * workgroup * 4 + RANK_BINS * 4 > LDS_BUDGET or _count_eqns(_jaxpr(eqn.params["body_jaxpr"])) < RANK_OPS:
+        return None
+    return _progress(eqn, env.producers)
+
+
+def _rank_in(mask: str) -> str:
+    """This lane's place among the set bits of a wavefront's `mask`."""
+    return (f"(int)__builtin_amdgcn_mbcnt_hi((unsigned int)({mask} >> 32), "
+            f"__builtin_amdgcn_mbcnt_lo((unsigned int){mask}, 0u))")
+
+
+RANK_PRELUDE = r"""
+/* The smallest bin (of 256) from which on at most `most` of the `live`
+   instances are counted, or 256 unless the quartiles lie at least `spread`
+   bins apart. Lane l sums bins 4 l .. 4 l + 3, then those of
+   the lanes above it; every wavefront gets the same answer. */
+__device__ __forceinline__ int ph_rank_cut(const unsigned int* hist, int live, int most, int spread) {
+    const int lane = (int)(threadIdx.x & 63u);
+    int c[4], above = 0;
+    for (int i = 0; i < 4; ++i) { c[i] = (int)hist[4 * lane + i]; above += c[i]; }
+    int sum = -above;
+    for (int off = 1; off < 64; off *= 2) {
+        const int up = __shfl_down(above, off);
+        above += lane + off < 64 ? up : 0;
+    }
+    sum += above;  /* in the bins of higher lanes */
+    int cut = 256, upper = 256, lower = 256;
+    for (int i = 3; i >= 0; --i) {
+        sum += c[i];
+        if (sum <= most) cut = 4 * lane + i;
+        if (4 * sum <= live) upper = 4 * lane + i;
+        if (4 * sum <= 3 * live) lower = 4 * lane + i;
+    }
+    for (int off = 32; off > 0; off /= 2) {
+        const int c2 = __shfl_xor(cut, off), u2 = __shfl_xor(upper, off), l2 = __shfl_xor(lower, off);
+        cut = c2 < cut ? c2 : cut;
+        upper = u2 < upper ? u2 : upper;
+        lower = l2 < lower ? l2 : lower;
+    }
+    return upper - lower >= spread ? cut : 256;
+}
+"""
 
 
 def emit_compacting_while(env: Any, cursor: Any, eqn: Any, emit_jaxpr: Any, declare_carries: Any,
@@ -243,7 +366,20 @@ def emit_compacting_while(env: Any, cursor: Any, eqn: Any, emit_jaxpr: Any, decl
     workgroup = env.compact_workgroup
     nw = workgroup // 64
     buf, res, cnt = cursor.fresh("_cbuf"), cursor.fresh("_cres"), cursor.fresh("_ccnt")
-    n_rows, kept_vals = _rows(state), [c for _, c in kept]
+    kept_vals = [c for _, c in kept]
+    ranked = _ranking(env, eqn, workgroup, _rows(state) + _rows(kept_vals) + 2)
+    if ranked is not None:
+        done = cursor.fresh("_done")
+        cursor.emit(f"unsigned int {done} = 0u;  // iterations this lane's instance has been given")
+        state = state + [dataclasses.replace(carries[0], expr=done, shape=(), ctype="unsigned int")]
+        hist, lcnt, limit, turn, due, look = (
+            cursor.fresh(p) for p in ("_chist", "_clong", "_climit", "_cturn", "_cdue", "_clook"))
+        cursor.emit(f"__shared__ unsigned int {hist}[{RANK_BINS}];")
+        cursor.emit(f"__shared__ int {lcnt}[{nw}];")
+        cursor.emit(f"if (threadIdx.x < {RANK_BINS}u) {hist}[threadIdx.x] = 0u;")
+        cursor.emit("__syncthreads();")
+        cursor.emit(f"int {limit} = {EPOCH}, {turn} = 0, {due} = 1;")
+    n_rows = _rows(state)
     cursor.emit(f"__shared__ unsigned int {buf}[{n_rows + 1}][{workgroup}];")
     if kept:
         cursor.emit(f"__shared__ unsigned int {res}[{_rows(kept_vals)}][{workgroup}];")
@@ -262,7 +398,7 @@ def emit_compacting_while(env: Any, cursor: Any, eqn: Any, emit_jaxpr: Any, decl
         # `unroll` iterations per pass, each with its own exit test (a break
         # in any of them leaves the epoch): the pass's counter and branch are
         # shared among them.
-        with cursor.block(f"for (int {ep} = 0; {ep} < {EPOCH}; {ep} += {unroll})"):
+        with cursor.block(f"for (int {ep} = 0; {ep} < {EPOCH if ranked is None else limit}; {ep} += {unroll})"):
             for _ in range(unroll):
                 (pred,) = emit_jaxpr(env, cursor, cj, cond_consts + carries)
                 live = cursor.fresh("_live")
@@ -281,6 +417,24 @@ def emit_compacting_while(env: Any, cursor: Any, eqn: Any, emit_jaxpr: Any, decl
                 for line in lines:
                     cursor.emit(line)
             cursor.emit(f"{slot} = -1;")
+        if ranked is not None:
+            from palladium_amd.emit.core import literal_cval
+
+            k, bound, start = ranked
+            edge = env.val(bound) if isinstance(bound, Literal) else cond_consts[cj.invars.index(bound)]
+            est, bin_ = cursor.fresh("_cest"), cursor.fresh("_cbin")
+            v = carries[k].at("0")
+            cursor.emit(f"{done} += (unsigned int){limit};")
+            cursor.emit(f"const bool {look} = ++{turn} >= {due};")
+            cursor.emit(f"int {bin_} = 0;")
+            with cursor.block(f"if ({look})"):
+                # Iterations left at the instance's average rate so far; NaN
+                # and no progress yet go to the last bin.
+                cursor.emit(f"const float {est} = ({edge.at('0')} - {v}) * (float){done}"
+                            f" * __builtin_amdgcn_rcpf({v} - {literal_cval(start, np.float32).expr});")
+                cursor.emit(f"{bin_} = {est} < 1.0f ? 0 : ({est} < {float(2 ** (RANK_BINS // 8 - 1)):.1f}f"
+                            f" ? (int)(__float_as_uint({est}) >> 20) - {127 * 8} : {RANK_BINS - 1});")
+                cursor.emit(f"if ({own}) atomicAdd(&{hist}[{bin_}], 1u);")
         mask, total, before, active = (cursor.fresh(p) for p in ("_cm", "_ctot", "_cbef", "_cact"))
         cursor.emit(f"const unsigned long long {mask} = __ballot({own});")
         with cursor.block("if ((threadIdx.x & 63u) == 0u)"):
@@ -294,11 +448,35 @@ def emit_compacting_while(env: Any, cursor: Any, eqn: Any, emit_jaxpr: Any, decl
         with cursor.block(f"if ({total} == 0)"):
             cursor.emit("break;")
         # Repack only when it frees a wavefront (the decision is uniform).
-        with cursor.block(f"if (({total} + 63) / 64 < {active})"):
+        repack = f"({total} + 63) / 64 < {active}"
+        place = f"{before} + {_rank_in(mask)}"
+        if ranked is not None:
+            rank, lmask, nlong, lbefore = (cursor.fresh(p) for p in ("_crank", "_clm", "_cnl", "_clb"))
+            cursor.emit(f"bool {rank} = false;")
+            cursor.emit(f"unsigned long long {lmask} = 0ull;")
+            cursor.emit(f"int {nlong} = 0, {lbefore} = 0;")
+            with cursor.block(f"if ({look} && {total} > {64 * RANK_WAVES})"):
+                cut = cursor.fresh("_ccut")
+                cursor.emit(f"const int {cut} = ph_rank_cut({hist}, {total}, {64 * RANK_WAVES}, {RANK_SPREAD});")
+                cursor.emit(f"{rank} = {cut} < {RANK_BINS};")
+                cursor.emit(f"{due} = {rank} ? {turn} + 1 : 4 * {turn};")
+                with cursor.block(f"if ({rank})"):
+                    cursor.emit(f"{lmask} = __ballot({own} && {bin_} >= {cut});")
+                    cursor.emit(f"if ((threadIdx.x & 63u) == 0u) {lcnt}[{wave}] = (int)__popcll({lmask});")
+                cursor.emit("__syncthreads();")  # also: every wave has read the histogram
+                w2 = cursor.fresh("_cw")
+                with cursor.block(f"for (int {w2} = 0; {rank} && {w2} < {nw}; ++{w2})"):
+                    cursor.emit(f"{nlong} += {lcnt}[{w2}]; {lbefore} += ({w2} < {wave}) ? {lcnt}[{w2}] : 0;")
+            with cursor.block("else"):
+                cursor.emit(f"{due} = {look} ? 2147483647 : {due};")  # not again: the count only falls
+            repack = f"{rank} || {repack}"
+            slow = f"({mask} & ~{lmask})"
+            place = (f"(({lmask} >> (threadIdx.x & 63u)) & 1ull) ? {lbefore} + {_rank_in(lmask)}"
+                     f" : {nlong} + ({before} - {lbefore}) + {_rank_in(slow)}")
+        with cursor.block(f"if ({repack})"):
             with cursor.block(f"if ({own})"):
                 pos = cursor.fresh("_cpos")
-                cursor.emit(f"const int {pos} = {before} + (int)__builtin_amdgcn_mbcnt_hi("
-                            f"(unsigned int)({mask} >> 32), __builtin_amdgcn_mbcnt_lo((unsigned int){mask}, 0u));")
+                cursor.emit(f"const int {pos} = {place};")
                 j = 0
                 for c in state:
                     lines, j = _store(buf, j, pos, c)
@@ -314,6 +492,12 @@ def emit_compacting_while(env: Any, cursor: Any, eqn: Any, emit_jaxpr: Any, decl
                 cursor.emit(f"{slot} = (int){buf}[{n_rows}][threadIdx.x];")
             with cursor.block("else"):
                 cursor.emit(f"{slot} = -1;")
+        if ranked is not None:
+            # The first waves, one on each SIMD, hold the instances with the
+            # most to do, and do more of their iterations an epoch.
+            cursor.emit(f"if ({look} && threadIdx.x < {RANK_BINS}u) {hist}[threadIdx.x] = 0u;")
+            cursor.emit(f"{limit} = {rank} && __builtin_amdgcn_readfirstlane({wave}) < {RANK_WAVES}"
+                        f" ? {EPOCH * RANK_TURNS} : {EPOCH};")
         # Nothing is written to LDS again before every lane has read.
         cursor.emit("__syncthreads();")
     # Every instance has finished: each lane takes its own back.

@@ -561,7 +561,7 @@ def emit_hip(spec: KernelSpec, kernel_name: str | None = None, block: int | None
         params.append(f"{qual}{ct}* __restrict__ arg{k}_base")
 
     body = plan.jaxpr if plan else spec.jaxpr
-    from palladium_amd.emit.compact import plan_for
+    from palladium_amd.emit.compact import RANK_PRELUDE, plan_for
     from palladium_amd.emit.optimize import fold_counters, funnel_shifts
 
     # The launch geometry was chosen on the traced jaxpr: a rewrite that
@@ -689,6 +689,7 @@ def emit_hip(spec: KernelSpec, kernel_name: str | None = None, block: int | None
 
     env.compact = body.eqns[cplan.index] if cplan is not None else None  # type: ignore[attr-defined]
     env.compact_workgroup = geo.block  # type: ignore[attr-defined]
+    env.compact_instances = geo.num_programs  # type: ignore[attr-defined]
     emit_jaxpr(env, cursor, body, ref_vals)
 
     head = (
@@ -700,6 +701,7 @@ def emit_hip(spec: KernelSpec, kernel_name: str | None = None, block: int | None
         [
             f"// palladium_amd kernel {name}: grid={grid} block={geo.block} blocks={geo.blocks} lanes={lanes}",
             PRELUDE,
+            *([RANK_PRELUDE] if any("ph_rank_cut" in line for line in cursor.lines) else []),
             *([SPREAD_PRELUDE] if spread is not None and (spread.reduces or spread.tile) else []),
             head,
             *cursor.lines,
