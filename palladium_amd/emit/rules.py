@@ -1017,7 +1017,14 @@ def _rule_lane_reduce(env: Environment, cursor: Cursor, eqn: JaxprEqn) -> None:
     cursor.emit(f"{wt} {acc} = ({wt})({src.at('0')});")
     off = _WAVE // 2
     while off >= 1:
-        cursor.emit(f"{acc} = {comb(acc, f'__shfl_xor({acc}, {off}, {_WAVE})')};")
+        other = f"__shfl_xor({acc}, {off}, {_WAVE})"
+        if not isf and kind in ("max", "min"):
+            # Exchanged outside of the choice: inside, only the lanes that
+            # take it would meet, and read what the others do not send.
+            name = cursor.fresh("_lx")
+            cursor.emit(f"const {wt} {name} = {other};")
+            other = name
+        cursor.emit(f"{acc} = {comb(acc, other)};")
         off //= 2
     if lanes > _WAVE:
         nw = lanes // _WAVE
