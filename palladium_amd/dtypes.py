@@ -20,6 +20,7 @@ rounding is innocuous).
 
 from __future__ import annotations
 
+import functools
 from typing import Any
 
 import numpy as np
@@ -57,7 +58,14 @@ def is_bf16(dt: Any) -> bool:
 
 def name(dt: Any) -> str:
     """The dtype's name, with the surrogate reporting "bfloat16"."""
-    return "bfloat16" if is_bf16(dt) else np.dtype(dt).name
+    return _name(dt) if isinstance(dt, np.dtype) else ("bfloat16" if is_bf16(dt) else np.dtype(dt).name)
+
+
+@functools.lru_cache(maxsize=64)
+def _name(d: np.dtype) -> str:
+    """NumPy builds a dtype's name anew at every look, and the emitter looks
+    at every operand of every operation."""
+    return "bfloat16" if d == bfloat16 or d.name == "bfloat16" else d.name
 
 
 def kind(dt: Any) -> str:

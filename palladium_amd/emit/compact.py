@@ -32,7 +32,7 @@ below a bound), each epoch ends with an estimate of its remaining iterations,
 (bound - carry) / progress per iteration so far; a histogram of the estimates
 in LDS gives the line above which the longest 256 lie, these move to the
 first four wavefronts (one a SIMD) and get three epochs' iterations to the
-others' one. The estimate only places instances: a wrong one costs time and
+others' one (four in SAFE). The estimate only places instances: a wrong one costs time and
 changes no result.
 
 Each instance runs exactly the operations it ran before, in the same
@@ -51,6 +51,7 @@ from __future__ import annotations
 
 import dataclasses
 import os
+import re
 from typing import Any
 
 import numpy as np
@@ -161,9 +162,9 @@ def workgroup_for(instances: int) -> int:
     SIMD pack best. Below, a large workgroup crowds its waves onto one CU
     while others stand empty: BS3 (REPRODUCIBLE, 2,646 attempts at most) in
     1,024 / 512 / 256 lanes takes 1,155 / 883 / 782 us at 65,536 instances and
-    1,132 / 869 / 778 at 5,000; with `_ranking` 1,024 / 512 lanes take 882 /
-    803 us at 131,072 and 892 / 1,004 at 262,144. Up to 4,096 instances the geometry is the
-    documented one, 1,024 lanes."""
+    1,132 / 869 / 778 at 5,000; ranked by progress (`_ranking`) 1,024 / 512
+    lanes take 882 / 803 us at 131,072 and 892 / 1,004 at 262,144. Up to 4,096
+    instances the geometry is the documented one, 1,024 lanes."""
     if instances <= 4096 or instances > 131_072:
         return WORKGROUP
     return 256 if instances <= 65_536 else 512
@@ -275,7 +276,10 @@ def _rows(vals: list) -> int:
 # the instances with the most to do, and their epochs in those of the others.
 RANK_BINS = 256
 RANK_WAVES = 4
-RANK_TURNS = 3
+# math mode -> epochs. BS3 in 2 / 3 / 4 of them: REPRODUCIBLE 946 / 851 / 865 us
+# at 262,144 instances, 3,710 / 3,378 / 3,412 at 1,048,576; SAFE, whose lone
+# wave is slower against four, 1,640 / 1,515 / 1,492 and 6,460 / 6,036 / 5,758.
+RANK_TURNS = {0: 4, 1: 3, 3: 3}
 # Ranked only while the estimates' quartiles lie this many bins apart: with
 # trip counts within 10 % of each other two or one bins would rank as well, and
 # cost 10-60 % (563 -> 637 us, 77 -> 129).
@@ -289,21 +293,45 @@ RANK_OPS = 64
 
 
 def _ranking(env: Any, eqn: Any, workgroup: int, rows: int) -> tuple | None:
-    """`_progress(eqn)` where ranking pays, else None: above 65,536 instances,
-    where a workgroup puts more than one wave on a SIMD, and with room in LDS
-    for the counts. BS3, REPRODUCIBLE / SAFE: 1,162 -> 902 / 1,927 -> 1,550 us
-    at 262,144 instances, 883 -> 805 / 1,399 -> 1,228 at 131,072 (workgroups
-    of 512), 4,590 -> 3,565 / 7,620 -> 6,157 at 1,048,576; three epochs against
-    two, four and six: 926 / 990 / 1,032 / 1,180 us. FAST keeps its order: its
-    text is held as a snapshot (672 -> 533 us when it is ranked)."""
+    """`_progress(eqn)` where ranking pays, else None: in workgroups of more
+    than 256 lanes, where a SIMD holds more than one wave, and with room in LDS
+    for the counts. BS3 unranked / ranked, REPRODUCIBLE and SAFE: 991 / 792 and
+    1,745 / 1,357 us at 1,000 instances, 782 / 692 and 1,343 / 1,149 at 131,072
+    (workgroups of 512), 1,065 / 851 and 1,864 / 1,492 at 262,144, 4,210 /
+    3,378 and 7,375 / 5,758 at 1,048,576. FAST keeps its order: its text is
+    held as a snapshot (672 -> 533 us when it is ranked)."""
     from palladium_amd.runtime import math_mode_ordinal
 
     mode = getattr(env, "math_mode", None)
-    if mode is None or math_mode_ordinal(mode) == 2 or env.compact_instances <= 65_536:
+    if mode is None or math_mode_ordinal(mode) not in RANK_TURNS or workgroup <= 256:
         return None
     if rows * workgroup * 4 + RANK_BINS * 4 > LDS_BUDGET or _count_eqns(_jaxpr(eqn.params["body_jaxpr"])) < RANK_OPS:
         return None
-    return _progress(eqn, env.producers)
+    found = _progress(eqn, env.producers)
+    return None if found is None else (*found, EPOCH * RANK_TURNS[math_mode_ordinal(mode)])
+
+
+# Functions with a branch for operands off their common path, by math mode; a
+# form without it adds the lanes that need it to a mask (emit/prelude.py). A
+# body with two of these branches or more runs on the common paths, with one
+# branch an iteration that leaves the state untaken; the rest of that epoch
+# then runs the full functions. A branch costs the lone wave its latency and
+# keeps the scheduler from overlapping what stands on both sides of it: BS3
+# REPRODUCIBLE (five branches -> one) 774 -> 692 us at 5,000 instances, 902 ->
+# 851 at 262,144, SAFE (three -> one) 1,184 -> 1,101 and 1,554 -> 1,515. With
+# one branch in the body there is nothing to merge. FAST has none.
+_CHECKED = {
+    0: re.compile(r"\bph_(?:pow|pow_log|pow_with_log)\("),
+    3: re.compile(r"\bph_(?:rdiv|rrcp|rpow|dlog2f|dexp2f|exp|log)\("),
+}
+
+
+def _checked(env: Any) -> Any:
+    """The pattern of such functions in this math mode, or None."""
+    from palladium_amd.runtime import math_mode_ordinal
+
+    mode = getattr(env, "math_mode", None)
+    return _CHECKED.get(math_mode_ordinal(mode)) if mode is not None else None
 
 
 def _rank_in(mask: str) -> str:
@@ -395,18 +423,53 @@ def emit_compacting_while(env: Any, cursor: Any, eqn: Any, emit_jaxpr: Any, decl
         cursor.emit(f"// {unroll} iterations per pass")
         from palladium_amd.emit.rules import select_guards
 
+        def iteration(odd: str | None) -> list[str]:
+            """One iteration, and its body's lines: with `odd`, on the common
+            paths of its checked functions, left untaken where a live lane
+            needs another."""
+            (pred,) = emit_jaxpr(env, cursor, cj, cond_consts + carries)
+            live = cursor.fresh("_live")
+            cursor.emit(f"const bool {live} = ({pred.at('0')}) && {slot} >= 0;")
+            # (the ballot of a bool tests the compare's own mask; __any goes
+            # through an int and a second compare)
+            none = f"!__any({live})" if odd is None else f"__builtin_amdgcn_ballot_w64({live}) == 0ull"
+            with cursor.block(f"if ({none})"):
+                cursor.emit("break;")
+            first = len(cursor.lines)
+            outs = emit_jaxpr(env, cursor, bj, body_consts + carries)
+            body = cursor.lines[first:]
+            if odd is not None:
+                name = cursor.fresh(odd)
+                cursor.lines[first:] = ["    " * cursor.indent + f"unsigned long long {name} = 0ull;",
+                                        *(names.sub(rf"\g<0>{name}, ", line) for line in body)]
+                with cursor.block(f"if (__builtin_expect(({name} & __builtin_amdgcn_ballot_w64({live})) != 0ull, 0))"):
+                    cursor.emit(f"{odd} = true;")
+                    cursor.emit("break;")
+            copy_back(cursor, outs, carries, predicate=live, guards=select_guards(env, bj, bn))
+            return body
+
+        trips = EPOCH if ranked is None else limit
+        names, odd, full = _checked(env), None, []
+        if names is not None:
+            # the rest of an epoch that met an odd lane
+            first = len(cursor.lines)
+            with cursor.block(f"for (; {ep} < {trips}; ++{ep})"):
+                body = iteration(None)
+            full = cursor.lines[first:]
+            del cursor.lines[first:]
+            if not any("{" in line for line in body) and sum(len(names.findall(line)) for line in body) >= 2:
+                odd = cursor.fresh("_odd")
+                cursor.emit(f"bool {odd} = false;")
+                cursor.emit(f"int {ep} = 0;")
         # `unroll` iterations per pass, each with its own exit test (a break
         # in any of them leaves the epoch): the pass's counter and branch are
         # shared among them.
-        with cursor.block(f"for (int {ep} = 0; {ep} < {EPOCH if ranked is None else limit}; {ep} += {unroll})"):
+        with cursor.block(f"for ({'' if odd else f'int {ep} = 0'}; {ep} < {trips}; {ep} += {unroll})"):
             for _ in range(unroll):
-                (pred,) = emit_jaxpr(env, cursor, cj, cond_consts + carries)
-                live = cursor.fresh("_live")
-                cursor.emit(f"const bool {live} = ({pred.at('0')}) && {slot} >= 0;")
-                with cursor.block(f"if (!__any({live}))"):
-                    cursor.emit("break;")
-                outs = emit_jaxpr(env, cursor, bj, body_consts + carries)
-                copy_back(cursor, outs, carries, predicate=live, guards=select_guards(env, bj, bn))
+                iteration(odd)
+        if odd is not None:
+            with cursor.block(f"if ({odd})"):
+                cursor.lines.extend(full)
         # Epoch boundary: the same condition, on the state as it stands.
         (pred,) = emit_jaxpr(env, cursor, cj, cond_consts + carries)
         cursor.emit(f"bool {own} = ({pred.at('0')}) && {slot} >= 0;")
@@ -420,7 +483,7 @@ def emit_compacting_while(env: Any, cursor: Any, eqn: Any, emit_jaxpr: Any, decl
         if ranked is not None:
             from palladium_amd.emit.core import literal_cval
 
-            k, bound, start = ranked
+            k, bound, start, long_epoch = ranked
             edge = env.val(bound) if isinstance(bound, Literal) else cond_consts[cj.invars.index(bound)]
             est, bin_ = cursor.fresh("_cest"), cursor.fresh("_cbin")
             v = carries[k].at("0")
@@ -497,7 +560,7 @@ def emit_compacting_while(env: Any, cursor: Any, eqn: Any, emit_jaxpr: Any, decl
             # most to do, and do more of their iterations an epoch.
             cursor.emit(f"if ({look} && threadIdx.x < {RANK_BINS}u) {hist}[threadIdx.x] = 0u;")
             cursor.emit(f"{limit} = {rank} && __builtin_amdgcn_readfirstlane({wave}) < {RANK_WAVES}"
-                        f" ? {EPOCH * RANK_TURNS} : {EPOCH};")
+                        f" ? {long_epoch} : {EPOCH};")
         # Nothing is written to LDS again before every lane has read.
         cursor.emit("__syncthreads();")
     # Every instance has finished: each lane takes its own back.

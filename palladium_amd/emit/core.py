@@ -689,7 +689,6 @@ def emit_hip(spec: KernelSpec, kernel_name: str | None = None, block: int | None
 
     env.compact = body.eqns[cplan.index] if cplan is not None else None  # type: ignore[attr-defined]
     env.compact_workgroup = geo.block  # type: ignore[attr-defined]
-    env.compact_instances = geo.num_programs  # type: ignore[attr-defined]
     emit_jaxpr(env, cursor, body, ref_vals)
 
     head = (

@@ -288,6 +288,24 @@ __device__ __forceinline__ float ph_pow_with_log(float x, float y, double lg) {
 }
 
 __device__ __forceinline__ float ph_pow(float x, float y) { return ph_pow_with_log(x, y, ph_pow_log(x)); }
+
+/* The common paths alone: what the function of the same name gives where no
+   lane needs its branch, whose lanes are added to `odd` instead. */
+__device__ __forceinline__ double ph_pow_log(unsigned long long& odd, float x) {
+    unsigned int ix = (__float_as_uint(x) & 0x7fffffffu) - 0x3f3504f4u;
+    odd |= ph_class_mask(x, 0x2f7);
+    return ph_log2_core((double)__uint_as_float((ix & 0x007fffffu) + 0x3f3504f4u), (int)ix >> 23);
+}
+
+__device__ __forceinline__ float ph_pow_with_log(unsigned long long& odd, float x, float y, double lg) {
+    double z = (double)y * lg;
+    odd |= ph_class_mask(x, 0x27f) | ph_outside_mask(z, -151.0, 129.0);
+    return (float)ph_exp2_dbl(z);
+}
+
+__device__ __forceinline__ float ph_pow(unsigned long long& odd, float x, float y) {
+    return ph_pow_with_log(odd, x, y, ph_pow_log(odd, x));
+}
 #endif
 #if PH_MATH_MODE == 3
 /* RN(1/b) for every float b. The hardware estimate (within 1 ulp) and one
@@ -441,6 +459,42 @@ __device__ __forceinline__ float ph_dlogf(float x) {
     if (__builtin_expect(ph_class_mask(x, 0x2ff) != 0ull, 0))
         r = __builtin_amdgcn_classf(x, 0x2ff) ? ph_dlogf_slow(x) : r;
     return r;
+}
+
+/* The common paths alone, as above. */
+__device__ __forceinline__ float ph_rrcp(unsigned long long& odd, float b) {
+    float y = __builtin_amdgcn_rcpf(b);
+    float e = __builtin_fmaf(-b, y, 1.0f);
+    y = __builtin_fmaf(e, y, y);
+    odd |= ph_class_mask(y, 0x2f7);
+    return y;
+}
+
+__device__ __forceinline__ float ph_rdiv(unsigned long long& odd, float a, float b) { return a * ph_rrcp(odd, b); }
+
+__device__ __forceinline__ float ph_dlog2f(unsigned long long& odd, float x) {
+    odd |= ph_class_mask(x, 0x2ff);
+    return (float)ph_rpow_log(x);
+}
+
+__device__ __forceinline__ float ph_dexp2f(unsigned long long& odd, float x) {
+    odd |= ph_wide_mask(x, 0x1p20f);
+    return (float)ph_rexp2((double)x);
+}
+
+__device__ __forceinline__ float ph_exp(unsigned long long& odd, float x) {
+    odd |= ph_wide_mask(x, 0x1p19f);
+    return (float)ph_rexp2((double)x * 1.4426950408889634);
+}
+
+__device__ __forceinline__ float ph_log(unsigned long long& odd, float x) {
+    odd |= ph_class_mask(x, 0x2ff);
+    return (float)(ph_rpow_log(x) * 0.6931471805599453);
+}
+
+__device__ __forceinline__ float ph_rpow(unsigned long long& odd, float x, float y) {
+    odd |= ph_class_mask(x, 0x2ff) | __builtin_amdgcn_ballot_w64(!(__builtin_fabsf(y) < 8192.0f));
+    return (float)ph_rexp2((double)y * ph_rpow_log(x));
 }
 
 /* Deterministic float sine and cosine. x = k pi/2 + r with |r| <= pi/4

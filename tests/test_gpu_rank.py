@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("kind", ["spread", "alike", "stuck"])
-@pytest.mark.parametrize("n", [65_537, 131_072, 140_001])
+@pytest.mark.parametrize("n", [1000, 4096, 65_537, 131_072, 140_001])
 def test_ranked_equals_the_plain_loop(monkeypatch, n, kind):
     print(f"[rank] n={n} {kind}", flush=True)
     r = steps(kind, n)

@@ -22,7 +22,7 @@ def test_ranked_loops(kwargs, want):
     assert _ranked(ranked_call(65_537, **kwargs), 65_537) is want
 
 
-@pytest.mark.parametrize("n, mode, want", [(65_536, "safe", False), (65_537, "safe", True), (131_073, "reproducible", True),
+@pytest.mark.parametrize("n, mode, want", [(4096, "safe", True), (65_536, "safe", False), (65_537, "safe", True), (131_073, "reproducible", True),
                                            (262_144, "fast", False)])
 def test_ranked_bs3(n, mode, want):
     assert _ranked(bs3_vdp_call(n, math_mode=mode), n, 3) is want
