@@ -90,6 +90,35 @@ __device__ __forceinline__ LVState lv_adv(LVState s, LVState k, float h) {
     LVState r; r.x = s.x + df_mul_f(k.x, h); r.y = s.y + df_mul_f(k.y, h); return r;
 }
 
+extern "C" __global__ void __launch_bounds__(256)
+lv_rk4_df32(const float* __restrict__ x0, const float* __restrict__ y0,
+            const float* __restrict__ a_, const float* __restrict__ b_,
+            const float* __restrict__ c_, const float* __restrict__ d_,
+            float* __restrict__ xo_hi, float* __restrict__ xo_lo,
+            float* __restrict__ yo_hi, float* __restrict__ yo_lo,
+            float dt, unsigned int steps, unsigned int n)
+{
+    const unsigned int i = blockIdx.x * 256u + threadIdx.x;
+    if (i >= n) return;
+    const float a = a_[i], b = b_[i], c = c_[i], d = d_[i];
+    const float half = 0.5f * dt, full = dt, sixth = dt / 6.0f;
+    LVState s; s.x = df_from_float(x0[i]); s.y = df_from_float(y0[i]);
+    for (unsigned int k = 0; k < steps; ++k) {
+        LVState k1 = lv_rhs(s, a, b, c, d);
+        LVState k2 = lv_rhs(lv_adv(s, k1, half), a, b, c, d);
+        LVState k3 = lv_rhs(lv_adv(s, k2, half), a, b, c, d);
+        LVState k4 = lv_rhs(lv_adv(s, k3, full), a, b, c, d);
+        LVState sum;
+        sum.x = k1.x + df_twice(k2.x) + df_twice(k3.x) + k4.x;
+        sum.y = k1.y + df_twice(k2.y) + df_twice(k3.y) + k4.y;
+        s = lv_adv(s, sum, sixth);
+    }
+    xo_hi[i] = s.x.hi; xo_lo[i] = s.x.lo;
+    yo_hi[i] = s.y.hi; yo_lo[i] = s.y.lo;
+}
+"""
+
+LV_DF32_PAIRS_SOURCE = DF32_PRELUDE + r"""
 /* Two lanes per trajectory, for ensembles of at most one wave per SIMD: a
    wave alone issues an instruction every 4 cycles, and its instruction count
    is the launch's time. The even lane holds x, the odd lane y. Both
@@ -114,14 +143,15 @@ __device__ __forceinline__ df32 lv_pair_rhs(df32 s, float p, float q) {
     y.hi = lv_odd(s.hi); y.lo = lv_odd(s.lo);
     return df_mul_f(s, p) - df_mul_f(x * y, q);
 }
-__device__ __forceinline__ void lv_pairs(
-            unsigned int t, const float* __restrict__ x0, const float* __restrict__ y0,
-            const float* __restrict__ a_, const float* __restrict__ b_,
-            const float* __restrict__ c_, const float* __restrict__ d_,
-            float* __restrict__ xo_hi, float* __restrict__ xo_lo,
-            float* __restrict__ yo_hi, float* __restrict__ yo_lo,
-            float dt, unsigned int steps, unsigned int n)
+extern "C" __global__ void __launch_bounds__(256)
+lv_rk4_df32_pairs(const float* __restrict__ x0, const float* __restrict__ y0,
+                  const float* __restrict__ a_, const float* __restrict__ b_,
+                  const float* __restrict__ c_, const float* __restrict__ d_,
+                  float* __restrict__ xo_hi, float* __restrict__ xo_lo,
+                  float* __restrict__ yo_hi, float* __restrict__ yo_lo,
+                  float dt, unsigned int steps, unsigned int n)
 {
+    const unsigned int t = blockIdx.x * 256u + threadIdx.x;
     const unsigned int i = t >> 1;
     if (i >= n) return;  /* both lanes of a pair */
     const bool odd = (t & 1u) != 0u;
@@ -137,38 +167,6 @@ __device__ __forceinline__ void lv_pairs(
     }
     (odd ? yo_hi : xo_hi)[i] = s.hi;
     (odd ? yo_lo : xo_lo)[i] = s.lo;
-}
-
-extern "C" __global__ void __launch_bounds__(256)
-lv_rk4_df32(const float* __restrict__ x0, const float* __restrict__ y0,
-            const float* __restrict__ a_, const float* __restrict__ b_,
-            const float* __restrict__ c_, const float* __restrict__ d_,
-            float* __restrict__ xo_hi, float* __restrict__ xo_lo,
-            float* __restrict__ yo_hi, float* __restrict__ yo_lo,
-            float dt, unsigned int steps, unsigned int n)
-{
-    const unsigned int t = blockIdx.x * 256u + threadIdx.x;
-    if (gridDim.x >= (2u * n + 255u) / 256u) {
-        lv_pairs(t, x0, y0, a_, b_, c_, d_, xo_hi, xo_lo, yo_hi, yo_lo, dt, steps, n);
-        return;
-    }
-    const unsigned int i = t;
-    if (i >= n) return;
-    const float a = a_[i], b = b_[i], c = c_[i], d = d_[i];
-    const float half = 0.5f * dt, full = dt, sixth = dt / 6.0f;
-    LVState s; s.x = df_from_float(x0[i]); s.y = df_from_float(y0[i]);
-    for (unsigned int k = 0; k < steps; ++k) {
-        LVState k1 = lv_rhs(s, a, b, c, d);
-        LVState k2 = lv_rhs(lv_adv(s, k1, half), a, b, c, d);
-        LVState k3 = lv_rhs(lv_adv(s, k2, half), a, b, c, d);
-        LVState k4 = lv_rhs(lv_adv(s, k3, full), a, b, c, d);
-        LVState sum;
-        sum.x = k1.x + df_twice(k2.x) + df_twice(k3.x) + k4.x;
-        sum.y = k1.y + df_twice(k2.y) + df_twice(k3.y) + k4.y;
-        s = lv_adv(s, sum, sixth);
-    }
-    xo_hi[i] = s.x.hi; xo_lo[i] = s.x.lo;
-    yo_hi[i] = s.y.hi; yo_lo[i] = s.y.lo;
 }
 """
 
@@ -196,6 +194,7 @@ LV_DF32_FLOPS_PER_STEP = (LV_DF32_MULS_PER_STEP * DF_MUL_FLOPS + LV_DF32_MUL_FS_
 PAIR_MAX = 32_768
 
 _kernel: rt.Kernel | None = None
+_pairs: rt.Kernel | None = None
 
 
 def lv_kernel() -> rt.Kernel:
@@ -206,12 +205,20 @@ def lv_kernel() -> rt.Kernel:
     return _kernel
 
 
+def lv_pairs_kernel() -> rt.Kernel:
+    """The same on two lanes per trajectory."""
+    global _pairs
+    if _pairs is None:
+        _pairs = rt.Kernel(LV_DF32_PAIRS_SOURCE, "lv_rk4_df32_pairs", rt.MathMode.SAFE)
+    return _pairs
+
+
 def lv_rk4_df32_device(bufs_in, bufs_out, dt: float, steps: int, n: int, stream=None) -> None:
     """Launch on device buffers: 6 inputs, 4 outputs (x_hi, x_lo, y_hi, y_lo).
-    Up to PAIR_MAX trajectories take two lanes each, which the kernel sees by
-    the launch's size."""
-    blocks = ((2 * n if n <= PAIR_MAX else n) + 255) // 256
-    lv_kernel().launch((blocks,), (256,), [*bufs_in, *bufs_out, np.float32(dt), np.uint32(steps), np.uint32(n)], stream)
+    Up to PAIR_MAX trajectories take two lanes each."""
+    kernel, lanes = (lv_pairs_kernel(), 2 * n) if n <= PAIR_MAX else (lv_kernel(), n)
+    kernel.launch(((lanes + 255) // 256,), (256,),
+                  [*bufs_in, *bufs_out, np.float32(dt), np.uint32(steps), np.uint32(n)], stream)
 
 
 def lv_rk4_df32(x0, y0, a, b, c, d, dt: float, steps: int):
