@@ -883,7 +883,7 @@ def _compacted_lane_fraction(attempts: np.ndarray) -> float:
     """Useful lane-iterations over issued ones under workgroup compaction:
     each epoch a 1,024-lane workgroup issues ceil(live / 64) wavefronts for
     EPOCH iterations (an upper bound: a wavefront leaves an epoch early
-    when all its lanes finish)."""
+    when all its lanes finish; instances in their own order, not ranked)."""
     from palladium_amd.emit.compact import EPOCH, WORKGROUP
 
     issued = 0
