@@ -200,6 +200,7 @@ CASES = {
        ((32, "f32"), (33, "f32"), (100, "f16"), (250, "bf16"), (1000, "u32"), (1025, "f32"), (1250, "bf16"),
         (4096, "i32"), (5001, "f32"), (300, "bool"), (2048, "f16"))},
     "flat_16_f32": flat(16, "f32"),
+    **{f"flat_one_{b}_f32": flat(b, "f32", grid=1) for b in (17, 1000, 4099)},
     "flat_wide_1024_f16": flat(1024, "f16", grid=2000),
     "flat_wide_f32": flat(1000, "f32", grid=1200),
     "flat_wide_bf16": flat(1000, "bf16", grid=2400),
