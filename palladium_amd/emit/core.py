@@ -465,6 +465,13 @@ def plan_of(spec: KernelSpec) -> Any:
     return memo["_spread_plan"] or lanes
 
 
+def _may_regroup(math_mode: Any) -> bool:
+    """Whether the mode's compiler options let operations be regrouped or fused."""
+    from palladium_amd.runtime import math_mode_ordinal
+
+    return math_mode is None or math_mode_ordinal(math_mode) in (1, 2)
+
+
 def _geometry(spec: KernelSpec, block: int | None, plan: Any) -> LaunchGeometry:
     """`plan`: what `plan_of` returned, or a lane count."""
     from palladium_amd.emit.lanes import workgroup_for
@@ -532,7 +539,7 @@ def emit_hip(spec: KernelSpec, kernel_name: str | None = None, block: int | None
     UnsupportedPrimitiveError
         A primitive with no registered rule.
     """
-    from palladium_amd.emit.prelude import PRELUDE, SPREAD_PRELUDE
+    from palladium_amd.emit.prelude import PRELUDE, ROUNDED_PRELUDE, SPREAD_PRELUDE
 
     from palladium_amd.emit.spread import SpreadPlan, spread_jaxpr, spread_prologue
 
@@ -638,6 +645,7 @@ def emit_hip(spec: KernelSpec, kernel_name: str | None = None, block: int | None
     if spread is not None:
         spread_prologue(env, cursor, spread, geo.block)
     env.lanes = lanes  # type: ignore[attr-defined]
+    env.rounded = spread is not None and spread.rounded and _may_regroup(math_mode)  # type: ignore[attr-defined]
     env.math_mode = math_mode  # type: ignore[attr-defined]
     env.grid = tuple(spec.grid)  # type: ignore[attr-defined]
     pid_vals = []
@@ -702,6 +710,7 @@ def emit_hip(spec: KernelSpec, kernel_name: str | None = None, block: int | None
             PRELUDE,
             *([RANK_PRELUDE] if any("ph_rank_cut" in line for line in cursor.lines) else []),
             *([SPREAD_PRELUDE] if spread is not None and (spread.reduces or spread.tile) else []),
+            *([ROUNDED_PRELUDE] if any("ph_bf16_" in line for line in cursor.lines) else []),
             head,
             *cursor.lines,
             "}",

@@ -642,3 +642,21 @@ __device__ __forceinline__ void ph_wave_sync() {
     __builtin_amdgcn_wave_barrier();
 }
 """
+
+# Only in kernels whose bfloat16 blocks are spread (emit/spread.py).
+ROUNDED_PRELUDE = r"""
+/* bfloat16 arithmetic that rounds every operation: no part of it is regrouped
+   or fused with a neighbour. FAST would make x * y + c * x into x * (y + c),
+   its sum rounded to 16 bits, or into an FMA in float32 (the options'
+   contraction ignores pragmas), so the value passes through an empty statement
+   that the compiler does not look into; it costs no instruction. */
+__device__ __forceinline__ __bf16 ph_round_bf16(__bf16 x) {
+    unsigned short u = __builtin_bit_cast(unsigned short, x);
+    asm("" : "+v"(u));
+    return __builtin_bit_cast(__bf16, u);
+}
+__device__ __forceinline__ __bf16 ph_bf16_add(float a, float b) { return ph_round_bf16((__bf16)(a + b)); }
+__device__ __forceinline__ __bf16 ph_bf16_sub(float a, float b) { return ph_round_bf16((__bf16)(a - b)); }
+__device__ __forceinline__ __bf16 ph_bf16_mul(float a, float b) { return ph_round_bf16((__bf16)(a * b)); }
+__device__ __forceinline__ __bf16 ph_bf16_div(float a, float b) { return ph_round_bf16((__bf16)(a / b)); }
+"""

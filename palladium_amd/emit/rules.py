@@ -209,6 +209,11 @@ def _reproducible(env: Environment) -> bool:
     return mode is not None and math_mode_ordinal(mode) == REPRODUCIBLE_ORDINAL
 
 
+# bfloat16 operations that FAST and RELAXED may regroup or fuse with their
+# neighbours: in `rounded` kernels by forms that round each (emit/prelude.py).
+ROUNDED = ("add", "sub", "mul", "div")
+
+
 def _rule_elementwise(env: Environment, cursor: Cursor, eqn: JaxprEqn) -> None:
     """All pure element-wise primitives (reference: `_rule_elementwise`,
     `src/palladium/emit/rules.py:274-351`). integer_pow expands to repeated
@@ -267,6 +272,8 @@ def _rule_elementwise(env: Environment, cursor: Cursor, eqn: JaxprEqn) -> None:
             recip = np.float32(1.0) / np.float32(eqn.invars[1].val)
             template = f"({{a}} * {format_float(float(recip))})"
             ops = ops[:1]
+    elif opname in ROUNDED and dst_ctype == BF16 and getattr(env, "rounded", False):
+        template = f"ph_bf16_{opname}({{a}}, {{b}})"
     else:
         template = _tmpl(opname, ops, dst_ctype)
 

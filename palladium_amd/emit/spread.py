@@ -87,6 +87,18 @@ MIN_SINGLE = 65
 # at 128 (SAFE, sums in order: 6.7 / 6.4, 9.3 / 6.6, 19.8 / 8.5); at 4 columns
 # a lane's row is one 16-byte load and both take 4.4.
 MIN_ROW = 8
+# Spread values are in registers, where FAST (and RELAXED's contraction) would
+# regroup bfloat16 arithmetic across operations: x * y + c * x becomes
+# x * (y + c), the sum rounded to 16 bits. One lane that held this many values
+# had them in memory, every operation rounded as the interpreter does, and
+# blocks of them still round so (`ROUNDED_PRELUDE`). Shorter ones were in
+# registers then too, as are the rows of a lane-parallel kernel. Results of
+# x * y + 0.1 x - y / (x^2 + 1) that differ from the one-lane form's, rounded /
+# regrouped: 28.9 / 0 % of them in blocks of 16, 18.5 / 7.6 of 24, 11.6 / 15.5
+# of 32, 0.4 / 26.2 of 48, 0 / 26.6 of 1,250, where the error against 64 bits is
+# 3.54e-3 / 3.63e-3 and the time the same. (float16 keeps the compiler's forms:
+# its error is no larger for them, 4.6e-4 against 5.5e-4 in blocks of 1,250.)
+MIN_ROUNDED = 32
 MAX_SLOTS = 64
 MAX_LANES = 1024
 WAVE = 64
@@ -127,6 +139,8 @@ class SpreadPlan:
     reduces: bool
     block: tuple[int, int]  # the block as traced (rows and width before flattening)
     tile: tuple[int, int] | None = None  # dots: 16 x 16 tiles down and across a wavefront's part
+
+    rounded: bool = False  # bfloat16 operations round one by one in every mode (`MIN_ROUNDED`)
 
     @property
     def lanes(self) -> int:
@@ -823,7 +837,8 @@ def spread_transform(spec: KernelSpec, lane_plan: Any = None) -> SpreadPlan | No
         if p.reduces:
             if max(1, DEFAULT_WORKGROUP // team) * row_stride(width) * 4 > ORDERED_LDS:
                 continue
-        return SpreadPlan(rows, width, team, slots, vec, p.reduces, (m, w))
+        return SpreadPlan(rows, width, team, slots, vec, p.reduces, (m, w),
+                          rounded=lane_plan is None and m * w >= MIN_ROUNDED)
     return None
 
 

@@ -47,3 +47,12 @@ def test_fast_close_to_the_interpreter(name):
         n = max(1, int(name.split("x")[1].split("_")[0])) if name.startswith(("rows", "dense_1", "dense_2")) else 64
         scale = np.abs(w).max() + np.sqrt(n)
         assert np.abs(g - w).max() <= 8 * eps * scale * np.sqrt(n)
+
+
+@pytest.mark.parametrize("mode", ["fast", "relaxed"])
+@pytest.mark.parametrize("name", ["flat_250_bf16", "flat_1250_bf16", "flat_wide_bf16"])
+def test_bfloat16_operations_round_one_by_one(name, mode):
+    """Sums and products rounded each: the interpreter's bits. (No operation
+    here leaves the exactly rounded ones, and no value is subnormal.)"""
+    for g, w in zip(*_run(name, mode)):
+        np.testing.assert_array_equal(g.view(np.uint16), w.view(np.uint16))

@@ -56,6 +56,17 @@ def test_compiles_without_scratch(name, mode):
     assert call.explain(*args).resources.scratch_bytes == 0
 
 
+@pytest.mark.parametrize("name, rounds", [("flat_250_bf16", True), ("flat_1250_bf16", True), ("flat_wide_bf16", True),
+                                          ("flat_100_f16", False), ("flat_5001_f32", False), ("rows_64x8_f32", False)])
+def test_bfloat16_operations_are_not_regrouped(name, rounds):
+    """Where one lane kept a block of bfloat16 values in memory, FAST and
+    RELAXED round every operation, as the interpreter does."""
+    for mode in ("fast", "relaxed"):
+        text = emit_hip(_spec(name), math_mode=mode)
+        assert all((f"= ph_bf16_{op}(" in text) == rounds for op in ("add", "mul", "sub"))
+    assert "ph_bf16_" not in emit_hip(_spec(name), math_mode="safe")
+
+
 def _row_call(kernel, m=4, w=64, out=None, **kw):
     s = pl.BlockSpec((m, w), lambda i: (i, 0))
     return pa.hip_call(kernel, grid=(3,), in_specs=[s], out_specs=s, out_shape=pl.ShapeDtypeStruct((3 * m, w), F), **kw)
