@@ -189,6 +189,7 @@ class _Pass:
         self.scopes: list[list] = []
         self.read: set[int] = set()  # output operands read back
         self.partial: set[int] = set()  # output operands not accessed element by own element
+        self.written: dict[int, set] = {}  # output operand -> its stores: (which lane, fixed indices)
         self.reduces = False
         self.whole = True  # only full-block accesses, no lone 'm' or 'w'
         self.spread_eqns = 0  # weighted by loop trips
@@ -537,6 +538,7 @@ class _Pass:
             if vary or (store and self.status(e.invars[1]) is not None and any(s != "u" for s in self.status(e.invars[1]))):
                 raise _Bail("part of the block")
             if store:
+                self.stored(k, (), indices)
                 used = e.outvars[0]
                 self.env[used], self.st[used] = None, None
                 v = e.invars[1]
@@ -572,6 +574,7 @@ class _Pass:
             self.emit(eqns, [self.env[ref], *leaves], [nv], "spread_get", params)
             self.bind(e.outvars[0], nv, st)
             return
+        self.stored(k, tuple((d, a) for d, a in zip(kept, axes) if a != "u"), indices)
         v = e.invars[1]
         s = self.status(v)
         x = self.atom(v)
@@ -596,6 +599,21 @@ class _Pass:
         self.env[old], self.st[old] = None, None
         self.emit(eqns, [self.env[ref], x, *leaves], [], "spread_swap", params)
         self.stores += 1
+
+    def stored(self, k: int, lane: tuple, indices: list) -> None:
+        """Note a store. The lane that stores an element follows from the
+        element and `lane`, the dims that lie along the block (none: lane 0
+        stores them all)."""
+        fixed = tuple(int(ix.val) if isinstance(ix, Literal) else int(ix) if isinstance(ix, (int, np.integer)) else None
+                      for ix in indices)
+        self.written.setdefault(k, set()).add((lane, fixed))
+
+    def overwrites(self) -> bool:
+        """Whether two lanes may store one element of an output. Nothing
+        orders their stores (an instance's lanes may lie in several
+        workgroups), so such a kernel keeps its program order in one lane."""
+        return any(a != b and not any(i is not None and j is not None and i != j for i, j in zip(at, bt))
+                   for stores in self.written.values() for a, at in stores for b, bt in stores)
 
     # -- control flow ---------------------------------------------------------
     def scan(self, e: JaxprEqn, eqns: list) -> None:
@@ -710,6 +728,8 @@ def _run(spec: KernelSpec, jaxpr: Jaxpr, m: int, w: int, slots: int, tiles: bool
     p.walk(jaxpr, eqns)
     if p.read & p.partial:
         raise _Bail("an output is read where another lane wrote it")
+    if p.overwrites():
+        raise _Bail("two lanes store one element of an output")
     return p, Jaxpr([], new, [], eqns)
 
 

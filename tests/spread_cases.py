@@ -221,3 +221,70 @@ CASES = {
     "two_dots_64x24x16": two_dots(64, 24, 16),
     **{f"single_{n}": single(n) for n in (65, 200, 1024, 3000)},
 }
+
+
+def overwritten(b, order):
+    """A block stored whole and in part, whose lanes would not be the same ones."""
+    one_d = not isinstance(b, tuple)
+
+    def kernel(x_ref, o_ref):
+        x = x_ref[...]
+
+        def whole():
+            o_ref[...] = x * 2.0
+
+        if order == "last":  # a boundary value after the block
+            whole()
+            if one_d:
+                o_ref[b - 1] = 5.0
+            else:
+                o_ref[b[0] - 1, b[1] - 1] = 5.0
+        elif order == "first":  # and before it
+            if one_d:
+                o_ref[b - 1] = 5.0
+            else:
+                o_ref[b[0] - 1, :] = x_ref[0, :]
+            whole()
+        elif order == "row":
+            whole()
+            o_ref[b[0] - 1, :] = x_ref[0, :]
+        elif order == "column":
+            whole()
+            o_ref[:, b[1] - 1] = x_ref[:, 0] + 1.0
+        elif order == "cross":  # a row and a column, without the block
+            o_ref[b[0] - 1, :] = x_ref[0, :]
+            o_ref[:, b[1] - 1] = x_ref[:, 0] + 1.0
+            o_ref[0, 0] = 3.0
+            o_ref[b[0] - 1, 0] = 7.0
+        elif order == "loop":
+            o_ref[...] = jnp.zeros((b,), jnp.float32)
+
+            def body(i, c):
+                o_ref[i * (b // 10)] = x_ref[i] + c
+                return c + 1.0
+
+            lax.fori_loop(0, 10, body, jnp.float32(0.0))
+        elif order == "branch":
+            whole()
+
+            def put(v):
+                o_ref[b - 2] = v
+                return v
+
+            lax.cond(x_ref[0] > 0.0, put, lambda v: v, jnp.float32(9.0))
+
+    def make(rng, grid=5, **kw):
+        shape = (b,) if one_d else b
+        s = pl.BlockSpec(shape, lambda i: (i, *(0,) * (len(shape) - 1)))
+        full = (grid * shape[0], *shape[1:])
+        call = pa.hip_call(kernel, grid=(grid,), in_specs=[s], out_specs=s, out_shape=pl.ShapeDtypeStruct(full, F), **kw)
+        return call, (_data(rng, full, "f32"),)
+
+    return make
+
+
+OVERWRITTEN = {f"{order}_{b if isinstance(b, int) else '%dx%d' % b}": overwritten(b, order) for order, b in
+               (("last", 100), ("last", 1000), ("first", 1000), ("loop", 1000), ("branch", 300), ("last", (8, 100)),
+                ("first", (8, 100)), ("row", (8, 100)), ("row", (300, 20)), ("column", (8, 100)), ("column", (3, 700)))}
+# The rest of the block is not written: compared where it is.
+CROSSED = {f"cross_{m}x{w}": overwritten((m, w), "cross") for m, w in ((8, 100), (20, 20))}

@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 from palladium_amd import dtypes
-from spread_cases import CASES
+from spread_cases import CASES, CROSSED, OVERWRITTEN
 
 pytestmark = pytest.mark.gpu
 
@@ -56,3 +56,19 @@ def test_bfloat16_operations_round_one_by_one(name, mode):
     here leaves the exactly rounded ones, and no value is subnormal.)"""
     for g, w in zip(*_run(name, mode)):
         np.testing.assert_array_equal(g.view(np.uint16), w.view(np.uint16))
+
+
+@pytest.mark.parametrize("mode", ["safe", "fast"])
+@pytest.mark.parametrize("name", sorted({**OVERWRITTEN, **CROSSED}))
+def test_later_stores_win(name, mode):
+    """Exact in both modes: one rounding an element."""
+    call, args = {**OVERWRITTEN, **CROSSED}[name](np.random.default_rng(7), math_mode=mode)
+    print(f"[spread] {name} {mode}", flush=True)
+    got, want = call(*args), call.interpret(*args)
+    if name in CROSSED:
+        m, w = (int(v) for v in name.split("_")[1].split("x"))
+        got, want = (v.reshape(5, m, w) for v in (got, want))
+        for at in ((slice(None), m - 1), (slice(None), slice(None), w - 1), (slice(None), 0, 0)):
+            np.testing.assert_array_equal(got[at], want[at])
+        return
+    np.testing.assert_array_equal(got, want)

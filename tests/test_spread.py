@@ -11,7 +11,7 @@ from palladium_amd.emit.core import plan_of
 from palladium_amd.emit.spread import MAX_LANES, MAX_SLOTS, SpreadPlan
 from palladium_amd.frontend import jnp, pl
 from palladium_amd.trace import trace
-from spread_cases import CASES
+from spread_cases import CASES, CROSSED, OVERWRITTEN
 
 F = np.float32
 
@@ -97,6 +97,25 @@ def test_other_forms_keep_their_lowering(kernel):
     spec = trace(_row_call(kernel)._staged, np.zeros((12, 64), F))
     assert not isinstance(plan_of(spec), SpreadPlan)
     emit_hip(spec, math_mode="fast")
+
+
+@pytest.mark.parametrize("name", sorted({**OVERWRITTEN, **CROSSED}))
+def test_stores_of_one_element_stay_in_one_lane(name):
+    """Lanes are not ordered: an element that two stores write has one lane."""
+    call, args = {**OVERWRITTEN, **CROSSED}[name](np.random.default_rng(1))
+    assert not isinstance(plan_of(trace(call._staged, *args)), SpreadPlan)
+
+
+def test_disjoint_stores_of_one_output_are_spread():
+    def kernel(x_ref, o_ref):
+        x = x_ref[...]
+        o_ref[:, 0] = jnp.sum(x, axis=1)  # both by the first lane of a row
+        o_ref[:, 1] = jnp.max(x, axis=1)
+        o_ref[3, 2] = 3.0  # by lane 0, another column
+
+    call = pa.hip_call(kernel, grid=(3,), in_specs=[pl.BlockSpec((4, 40), lambda i: (i, 0))],
+                       out_specs=pl.BlockSpec((4, 3), lambda i: (i, 0)), out_shape=pl.ShapeDtypeStruct((12, 3), F))
+    assert isinstance(plan_of(trace(call._staged, np.zeros((12, 40), F))), SpreadPlan)
 
 
 def test_small_blocks_and_plain_gridless_calls_keep_one_lane():
