@@ -16,7 +16,10 @@ emission:
   is done by lane 0 only;
 - `iota` along the lane dim is the lane id;
 - a reduction over the lane dim becomes a cross-lane reduction
-  (`lane_reduce_*`: wavefront shuffles, then LDS across the instance's waves).
+  (`lane_reduce_*`: wavefront shuffles, then LDS across the instance's waves);
+- an output whose elements have several lanes (rows by their own, and a row or
+  element by lane 0 or read by all) is accessed between `lane_sync`s, which keep
+  the program's order among the instance's lanes.
 
 Control flow stays uniform within an instance (loop conditions and switch
 indices have no lane dim), so every lane of an instance takes the same path
@@ -119,9 +122,13 @@ def _iota_rows(j: Jaxpr) -> int | None:
 
 
 class _Pass:
-    def __init__(self, b: int):
+    def __init__(self, b: int, ordered: frozenset[int] = frozenset()):
         self.b = b
         self.lane_var: Var | None = None
+        self.operand: dict[Any, int] = {}  # ref -> operand
+        self.ordered = ordered  # operands whose accesses by lane 0 and by all lanes are synchronised
+        self.accesses: dict[int, set[str]] = {}  # operand -> "row", "row=", "one=" and "all" (= stores)
+        self.used: set[Any] = set()
 
     # -- helpers -----------------------------------------------------------
     def per_lane(self, aval: Any, st: str) -> Any:
@@ -131,6 +138,28 @@ class _Pass:
 
     def status_of_shape(self, aval: Any) -> bool:
         return not isinstance(aval, (KeyAval, RefAval)) and len(aval.shape) >= 1 and aval.shape[0] == self.b
+
+    def refs(self, inner: list, outer: list) -> None:
+        for v, x in zip(inner, outer):
+            if not isinstance(x, Literal) and x in self.operand:
+                self.operand[v] = self.operand[x]
+
+    def access(self, ref: Any, kind: str) -> None:
+        self.accesses.setdefault(self.operand[ref], set()).add(kind)
+
+    def mixed(self) -> frozenset[int]:
+        """Operands of which a lane reads or overwrites what another stores."""
+        return frozenset(k for k, kinds in self.accesses.items()
+                         if "one=" in kinds and kinds - {"one="} or "row=" in kinds and "all" in kinds)
+
+    def whole(self, e: JaxprEqn, out: Any) -> None:
+        """An access that is not each lane's own row: lane 0 stores, every
+        lane loads."""
+        store = e.primitive.name == "swap"
+        if store and e.outvars[0] in self.used:
+            raise _Bail("a store by lane 0 that returns the value before it")
+        self.access(e.invars[0], "one=" if store else "all")
+        out(U, params={**e.params, "lane0_only": True} if store else None, sync=self.operand[e.invars[0]] in self.ordered)
 
     def lane(self, eqns: list[JaxprEqn]) -> Var:
         v = Var(ShapedArray((), "int32"))
@@ -158,6 +187,9 @@ class _Pass:
             return U if isinstance(x, Literal) else st[x]
 
         for e in j.eqns:
+            self.used.update(x for x in e.invars if isinstance(x, Var))
+        self.used.update(o for o in j.outvars if isinstance(o, Var))
+        for e in j.eqns:
             self.eqn(e, env, st, eqns, a, s_of, ref_lane)
         outs = [a(o) for o in j.outvars]
         return Jaxpr([], new_invars, outs, eqns), [s_of(o) for o in j.outvars]
@@ -166,7 +198,8 @@ class _Pass:
         name = e.primitive.name
         ins_st = [s_of(x) for x in e.invars]
 
-        def out(status: str, params: dict | None = None, invars: list | None = None, prim: str | None = None) -> None:
+        def out(status: str, params: dict | None = None, invars: list | None = None, prim: str | None = None,
+                sync: bool = False) -> None:
             nouts = []
             for ov in e.outvars:
                 if status == L and not self.status_of_shape(ov.aval):
@@ -175,8 +208,10 @@ class _Pass:
                 env[ov] = nv
                 st[ov] = status
                 nouts.append(nv)
-            eqns.append(JaxprEqn(invars if invars is not None else [a(x) for x in e.invars], nouts,
-                                 primitive(prim or name), params if params is not None else dict(e.params)))
+            new = JaxprEqn(invars if invars is not None else [a(x) for x in e.invars], nouts,
+                           primitive(prim or name), params if params is not None else dict(e.params))
+            fence = [JaxprEqn([], [], primitive("lane_sync"), {"lanes": self.b})] if sync else []
+            eqns.extend([*fence, new, *fence])
 
         if name in _ELEMENTWISE:
             if L in ins_st:
@@ -198,10 +233,7 @@ class _Pass:
             if not is_lane_ref:
                 if name == "swap" and s_of(e.invars[1]) == L:
                     raise _Bail("lane value stored to a non-lane ref")
-                params = dict(e.params)
-                if name == "swap":
-                    params["lane0_only"] = True
-                out(U, params=params)
+                self.whole(e, out)
                 return
             if not idx:
                 indices = [Slice(0, n, 1) for n in env[ref].aval.shape]
@@ -211,11 +243,9 @@ class _Pass:
             if not (isinstance(first, Slice) and isinstance(first.start, int) and first.start == 0 and first.size == self.b):
                 if name == "swap" and s_of(e.invars[1]) == L:
                     raise _Bail("lane value stored to a single row")
-                params = dict(e.params)
-                if name == "swap":
-                    params["lane0_only"] = True
-                out(U, params=params)
+                self.whole(e, out)
                 return
+            self.access(ref, "row=" if name == "swap" else "row")
             lane = self.lane(eqns)
             leaves: list[Any] = [lane]
             tmpl: list[Any] = [_Leaf(0)]
@@ -336,6 +366,7 @@ class _Pass:
         if name in ("pjit", "jit", "closed_call", "core_call", "custom_jvp_call", "custom_vjp_call"):
             inner = e.params.get("jaxpr") or e.params.get("call_jaxpr")
             body = getattr(inner, "jaxpr", inner)
+            self.refs(body.invars, e.invars[-len(body.invars):])
             nb, outs_st = self.jaxpr(body, ins_st[-len(body.invars):], dict(ref_lane))
             self._bind_outs(e, env, st, eqns, outs_st, "pjit", {"jaxpr": ClosedJaxpr(nb, [])},
                             [a(x) for x in e.invars][-len(body.invars):])
@@ -345,6 +376,7 @@ class _Pass:
             nc = len(e.outvars)
             nconst = len(e.invars) - nc
             carry_st = ins_st[nconst:]
+            self.refs(body.invars, e.invars)
             for _ in range(len(carry_st) + 1):
                 nb, outs_st = self.jaxpr(body, ins_st[:nconst] + carry_st, dict(ref_lane))
                 merged = [L if L in (c, o) else U for c, o in zip(carry_st, outs_st)]
@@ -362,6 +394,8 @@ class _Pass:
             cj = getattr(e.params["cond_jaxpr"], "jaxpr", e.params["cond_jaxpr"])
             bj = getattr(e.params["body_jaxpr"], "jaxpr", e.params["body_jaxpr"])
             carry_st = ins_st[cn + bn:]
+            self.refs(cj.invars, e.invars[:cn])
+            self.refs(bj.invars, e.invars[cn:])
             for _ in range(len(carry_st) + 1):
                 nb, outs_st = self.jaxpr(bj, ins_st[cn:cn + bn] + carry_st, dict(ref_lane))
                 merged = [L if L in (c, o) else U for c, o in zip(carry_st, outs_st)]
@@ -382,6 +416,8 @@ class _Pass:
             if ins_st[0] == L:
                 raise _Bail("cond index varies across lanes")
             branches = e.params["branches"]
+            for br in branches:
+                self.refs(getattr(br, "jaxpr", br).invars, e.invars[1:])
             results = [self.jaxpr(getattr(br, "jaxpr", br), ins_st[1:], dict(ref_lane)) for br in branches]
             outs_st = [L if any(r[1][k] == L for r in results) else U for k in range(len(e.outvars))]
             for r in results:
@@ -418,12 +454,20 @@ def _lane_transform(spec: KernelSpec) -> LanePlan | None:
     if found is None:
         return None
     b, lane_ops = found
-    p = _Pass(b)
-    ref_lane: dict[Any, bool] = {}
-    for k, v in enumerate(spec.jaxpr.invars):
-        ref_lane[v] = k in lane_ops
+
+    def run(ordered: frozenset[int] = frozenset()) -> tuple[_Pass, Jaxpr]:
+        p = _Pass(b, ordered)
+        ref_lane: dict[Any, bool] = {}
+        for k, v in enumerate(spec.jaxpr.invars):
+            ref_lane[v] = k in lane_ops
+            p.operand[v] = k
+        return p, p.jaxpr(spec.jaxpr, [U] * len(spec.jaxpr.invars), ref_lane)[0]
+
     try:
-        nj, _ = p.jaxpr(spec.jaxpr, [U] * len(spec.jaxpr.invars), ref_lane)
+        p, nj = run()
+        mixed = p.mixed()
+        if mixed:
+            _, nj = run(mixed)
     except _Bail:
         return None
     rows = _ragged_rows(spec, b, lane_ops, nj)

@@ -998,6 +998,18 @@ def _rule_lane_index(env: Environment, cursor: Cursor, eqn: JaxprEqn) -> None:
 _WAVE = 64
 
 
+@rule("lane_sync")
+def _rule_lane_sync(env: Environment, cursor: Cursor, eqn: JaxprEqn) -> None:
+    """The instance's lanes see each other's accesses before this point. An
+    instance of more than a wavefront is a workgroup; one wavefront's accesses
+    run in order, so only the compiler has to keep them so."""
+    if int(eqn.params["lanes"]) > _WAVE:
+        cursor.emit("__syncthreads();")
+        return
+    cursor.emit('__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");')
+    cursor.emit("__builtin_amdgcn_wave_barrier();")
+
+
 @rule("lane_reduce")
 def _rule_lane_reduce(env: Environment, cursor: Cursor, eqn: JaxprEqn) -> None:
     """Reduce one scalar per lane over the instance's lanes; every lane gets

@@ -288,3 +288,33 @@ OVERWRITTEN = {f"{order}_{b if isinstance(b, int) else '%dx%d' % b}": overwritte
                 ("first", (8, 100)), ("row", (8, 100)), ("row", (300, 20)), ("column", (8, 100)), ("column", (3, 700)))}
 # The rest of the block is not written: compared where it is.
 CROSSED = {f"cross_{m}x{w}": overwritten((m, w), "cross") for m, w in ((8, 100), (20, 20))}
+
+
+def read_by_all(b):
+    """An output's element read by every lane after lane 0 stored it, its
+    rows summed one by one after each lane stored its own."""
+    def kernel(x_ref, o_ref, s_ref):
+        s_ref[0] = jnp.max(x_ref[...])
+        o_ref[...] = x_ref[...] - s_ref[0]
+        s_ref[1] = o_ref[b - 1] * 2.0
+
+        def body(i, c):
+            s_ref[1] = s_ref[1] + o_ref[i * (b // 8)]
+            return c
+
+        lax.fori_loop(0, 8, body, jnp.float32(0.0))
+
+    def make(rng, grid=5, **kw):
+        s = pl.BlockSpec((b,), lambda i: (i,))
+        call = pa.hip_call(kernel, grid=(grid,), in_specs=[s], out_specs=(s, pl.BlockSpec((2,), lambda i: (i,))),
+                           out_shape=(pl.ShapeDtypeStruct((grid * b,), F), pl.ShapeDtypeStruct((grid * 2,), F)), **kw)
+        return call, (_data(rng, grid * b, "f32"),)
+
+    return make
+
+
+# The same where a block's rows have a lane each.
+LANE_ROWS = {**{f"{order}_{b if isinstance(b, int) else '%dx%d' % b}": overwritten(b, order) for order, b in
+                (("last", 64), ("last", 256), ("first", 1024), ("loop", 256), ("branch", 128), ("last", (128, 4)),
+                 ("first", (128, 4)), ("row", (256, 3)), ("row", (64, 3)))},
+             **{f"read_by_all_{b}": read_by_all(b) for b in (64, 256, 1024)}}

@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 from palladium_amd import dtypes
-from spread_cases import CASES, CROSSED, OVERWRITTEN
+from spread_cases import CASES, CROSSED, LANE_ROWS, OVERWRITTEN
 
 pytestmark = pytest.mark.gpu
 
@@ -72,3 +72,14 @@ def test_later_stores_win(name, mode):
             np.testing.assert_array_equal(got[at], want[at])
         return
     np.testing.assert_array_equal(got, want)
+
+
+@pytest.mark.parametrize("mode", ["safe", "fast"])
+@pytest.mark.parametrize("name", sorted(LANE_ROWS))
+def test_lanes_of_an_instance_keep_its_order(name, mode):
+    """Exact in both modes: one rounding an operation, sums in their order."""
+    call, args = LANE_ROWS[name](np.random.default_rng(7), math_mode=mode)
+    print(f"[lanes] {name} {mode}", flush=True)
+    got, want = call(*args), call.interpret(*args)
+    for g, w in zip(*((v,) if isinstance(v, np.ndarray) else v for v in (got, want))):
+        np.testing.assert_array_equal(g, w)

@@ -8,10 +8,11 @@ import pytest
 import palladium_amd as pa
 from palladium_amd.emit import emit_hip, launch_geometry
 from palladium_amd.emit.core import plan_of
+from palladium_amd.emit.lanes import LanePlan
 from palladium_amd.emit.spread import MAX_LANES, MAX_SLOTS, SpreadPlan
 from palladium_amd.frontend import jnp, pl
 from palladium_amd.trace import trace
-from spread_cases import CASES, CROSSED, OVERWRITTEN
+from spread_cases import CASES, CROSSED, LANE_ROWS, OVERWRITTEN
 
 F = np.float32
 
@@ -104,6 +105,41 @@ def test_stores_of_one_element_stay_in_one_lane(name):
     """Lanes are not ordered: an element that two stores write has one lane."""
     call, args = {**OVERWRITTEN, **CROSSED}[name](np.random.default_rng(1))
     assert not isinstance(plan_of(trace(call._staged, *args)), SpreadPlan)
+
+
+@pytest.mark.parametrize("name", sorted(LANE_ROWS))
+def test_lane_rows_are_synchronised_where_lanes_meet(name):
+    """Lane 0's stores, and what every lane reads, stand between barriers
+    (of the wavefront, where it is the whole instance)."""
+    call, args = LANE_ROWS[name](np.random.default_rng(1))
+    spec = trace(call._staged, *args)
+    plan = plan_of(spec)
+    assert isinstance(plan, LanePlan)
+    lines = emit_hip(spec, math_mode="safe").split('extern "C"')[-1].splitlines()
+    sync = ("__syncthreads();",) if plan.lanes > 64 else ("__builtin_amdgcn_wave_barrier();",
+                                                          '__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");')
+    guards = [i for i, x in enumerate(lines) if x.lstrip().startswith("if (_lane == 0) {")]
+    assert guards
+    for i in guards:
+        end = next(j for j in range(i, len(lines)) if lines[j] == lines[i].replace("if (_lane == 0) {", "}"))
+        assert lines[i - 1].strip() in sync and lines[end + 1].strip() in sync
+
+
+def test_lane_rows_of_their_own_need_no_barrier():
+    def kernel(x_ref, o_ref, s_ref):
+        x = x_ref[...]
+        o_ref[...] = x
+        o_ref[...] = o_ref[...] * 2.0
+        s_ref[0] = 1.0
+        s_ref[1] = 2.0
+
+    s = pl.BlockSpec((128, 2), lambda i: (i, 0))
+    call = pa.hip_call(kernel, grid=(4,), in_specs=[s], out_specs=(s, pl.BlockSpec((2,), lambda i: (i,))),
+                       out_shape=(pl.ShapeDtypeStruct((512, 2), F), pl.ShapeDtypeStruct((8,), F)))
+    spec = trace(call._staged, np.zeros((512, 2), F))
+    assert isinstance(plan_of(spec), LanePlan)
+    text = emit_hip(spec, math_mode="safe")
+    assert "__syncthreads" not in text and "wave_barrier" not in text
 
 
 def test_disjoint_stores_of_one_output_are_spread():
