@@ -189,6 +189,7 @@ class _Pass:
         self.scopes: list[list] = []
         self.read: set[int] = set()  # output operands read back
         self.partial: set[int] = set()  # output operands not accessed element by own element
+        self.used: set[Var] = set()  # values something reads
         self.written: dict[int, set] = {}  # output operand -> its stores: (which lane, fixed indices)
         self.reduces = False
         self.whole = True  # only full-block accesses, no lone 'm' or 'w'
@@ -284,6 +285,7 @@ class _Pass:
         for o in j.outvars:
             if isinstance(o, Var):
                 uses.setdefault(o, []).append(("out", 0))
+        self.used.update(uses)
         for e in j.eqns:
             if e.primitive.name == "get" and uses.get(e.outvars[0]) and all(
                     n == "dot_general" for n, _ in uses[e.outvars[0]]) and self.whole_input(e):
@@ -515,6 +517,8 @@ class _Pass:
         ref = e.invars[0]
         k = self.refs[ref]
         shape = tuple(int(d) for d in ref.aval.shape)
+        if store and e.outvars[0] in self.used:
+            raise _Bail("a store's value before it")
         idx = e.params["tree"].unflatten(list(e.invars[2 if store else 1:]))
         indices = list(idx[0].indices) if idx else [Slice(0, n, 1) for n in shape]
         kept = [d for d, ix in enumerate(indices) if isinstance(ix, Slice)]

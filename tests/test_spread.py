@@ -11,6 +11,8 @@ from palladium_amd.emit.core import plan_of
 from palladium_amd.emit.lanes import LanePlan
 from palladium_amd.emit.spread import MAX_LANES, MAX_SLOTS, SpreadPlan
 from palladium_amd.frontend import jnp, pl
+from palladium_amd.frontend.core import current_builder
+from palladium_amd.ir import ShapedArray
 from palladium_amd.trace import trace
 from spread_cases import CASES, CROSSED, LANE_ROWS, OVERWRITTEN
 
@@ -91,10 +93,18 @@ def _part(x_ref, o_ref):
     o_ref[2:4, :] = x_ref[2:4, :]
 
 
-@pytest.mark.parametrize("kernel", [_read_back, _across_rows, _transposed, _part])
+def _exchange(x_ref, o_ref):
+    """A store that returns what the block held."""
+    o_ref[...] = x_ref[...]
+    tree, leaves = o_ref._indexer(...)
+    (old,) = current_builder().add("swap", [o_ref._t, x_ref[...] * 2.0, *leaves], [ShapedArray((4, 64), F)], tree=tree)
+    o_ref[...] = old + 1.0
+
+
+@pytest.mark.parametrize("kernel", [_read_back, _across_rows, _transposed, _part, _exchange])
 def test_other_forms_keep_their_lowering(kernel):
     """An output read where another lane wrote it, a reduction across rows,
-    a transpose, part of a block."""
+    a transpose, part of a block, a store whose old value is used."""
     spec = trace(_row_call(kernel)._staged, np.zeros((12, 64), F))
     assert not isinstance(plan_of(spec), SpreadPlan)
     emit_hip(spec, math_mode="fast")
