@@ -94,11 +94,10 @@ def _part(x_ref, o_ref):
 
 
 def _exchange(x_ref, o_ref):
-    """A store that returns what the block held."""
-    o_ref[...] = x_ref[...]
-    tree, leaves = o_ref._indexer(...)
-    (old,) = current_builder().add("swap", [o_ref._t, x_ref[...] * 2.0, *leaves], [ShapedArray((4, 64), F)], tree=tree)
-    o_ref[...] = old + 1.0
+    """A store that returns what the element held."""
+    tree, leaves = o_ref._indexer((0, 0))
+    (old,) = current_builder().add("swap", [o_ref._t, x_ref[0, 0] * 2.0, *leaves], [ShapedArray((), F)], tree=tree)
+    o_ref[...] = x_ref[...] + old
 
 
 @pytest.mark.parametrize("kernel", [_read_back, _across_rows, _transposed, _part, _exchange])
