@@ -541,7 +541,7 @@ def emit_hip(spec: KernelSpec, kernel_name: str | None = None, block: int | None
     """
     from palladium_amd.emit.prelude import PRELUDE, ROUNDED_PRELUDE, SPREAD_PRELUDE
 
-    from palladium_amd.emit.spread import SpreadPlan, spread_jaxpr, spread_prologue
+    from palladium_amd.emit.spread import SpreadPlan, spread_jaxpr, spread_prologue, staging
 
     name = kernel_name or spec.name
     plan = plan_of(spec)
@@ -712,6 +712,7 @@ def emit_hip(spec: KernelSpec, kernel_name: str | None = None, block: int | None
             *([SPREAD_PRELUDE] if spread is not None and (spread.reduces or spread.tile) else []),
             *([ROUNDED_PRELUDE] if any("ph_bf16_" in line for line in cursor.lines) else []),
             head,
+            *staging(env),
             *cursor.lines,
             "}",
             "",

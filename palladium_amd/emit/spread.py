@@ -105,6 +105,7 @@ WAVE = 64
 TILE = 16
 # Ordered sums stage a team's row in LDS: at most this much per workgroup.
 ORDERED_LDS = 60 * 1024
+STAGING = "_rows"
 DEFAULT_WORKGROUP = 256
 
 
@@ -808,6 +809,12 @@ def _layout(p: _Pass, m: int, w: int, programs: int) -> tuple[int, int, int] | N
     return (team, slots, v) if slots <= MAX_SLOTS else None
 
 
+def staging(env: Environment) -> list[str]:
+    """The kernel's array for the rows of ordered sums, if it has any."""
+    n = getattr(env, "staged", 0)
+    return [f"    __shared__ __attribute__((aligned(16))) unsigned char {STAGING}[{n}];"] if n else []
+
+
 def own_rules() -> bool:
     """Whether the rules this lowering stands in for are the built-in ones
     (a user's own rule for an access or a reduction keeps its say)."""
@@ -1226,11 +1233,13 @@ def _ordered_sum(env: Environment, cursor: Cursor, plan: SpreadPlan, src: CVal, 
     act = "float" if ct == "__bf16" else ct
     stride = row_stride(plan.width)
     teams = max(1, env.spread_block // plan.team)  # type: ignore[attr-defined]
-    sh, row, acc = cursor.fresh("_row"), cursor.fresh("_rp"), cursor.fresh("_acc")
+    row, acc = cursor.fresh("_rp"), cursor.fresh("_acc")
     sync = "__syncthreads();" if plan.team > WAVE else "ph_wave_sync();"
-    cursor.emit(f"__shared__ __attribute__((aligned(16))) {act} {sh}[{teams} * {stride}];")
+    # One array for all sums of a kernel (each ends with its reads done): the
+    # compiler adds up those of a kernel, and three of 58 KB are past the CU's.
+    env.staged = max(getattr(env, "staged", 0), teams * stride * (2 if act == "_Float16" else 4))  # type: ignore[attr-defined]
     at = f"(threadIdx.x / {plan.team}u) * {stride}u" if teams > 1 else "0"
-    cursor.emit(f"{act}* {row} = {sh} + {at};")
+    cursor.emit(f"{act}* {row} = ({act}*){STAGING} + {at};")
     for s in range(plan.slots):
         q = s // plan.vec
         put = f"{row}[_w{q} + {s % plan.vec}] = ({act})({src.at(str(s))});"

@@ -318,3 +318,29 @@ LANE_ROWS = {**{f"{order}_{b if isinstance(b, int) else '%dx%d' % b}": overwritt
                 (("last", 64), ("last", 256), ("first", 1024), ("loop", 256), ("branch", 128), ("last", (128, 4)),
                  ("first", (128, 4)), ("row", (256, 3)), ("row", (64, 3)))},
              **{f"read_by_all_{b}": read_by_all(b) for b in (64, 256, 1024)}}
+
+
+def moments(m, w, n, dt="f32"):
+    """n sums along each row, one after another, in two accumulation types."""
+    def kernel(x_ref, o_ref, n_ref):
+        x = x_ref[...]
+        z = x
+        for _ in range(n):
+            z = x - jnp.sum(z, axis=1, keepdims=True) * 0.125
+        o_ref[...] = z
+        n_ref[...] = jnp.sum(jnp.where(z > x, 0.5, 0.25), axis=1)
+
+    def make(rng, grid=3, **kw):
+        s = pl.BlockSpec((m, w), lambda i: (i, 0))
+        call = pa.hip_call(kernel, grid=(grid,), in_specs=[s], out_specs=(s, pl.BlockSpec((m,), lambda i: (i,))),
+                           out_shape=(pl.ShapeDtypeStruct((grid * m, w), _DT[dt]),
+                                      pl.ShapeDtypeStruct((grid * m,), F)), **kw)
+        return call, (_data(rng, (grid * m, w), dt),)
+
+    return make
+
+
+# Together past a workgroup's LDS, were each staged by itself.
+MOMENTS = {f"moments_{m}x{w}_{n}_{dt}": moments(m, w, n, dt) for m, w, n, dt in
+           ((64, 900, 3, "f32"), (64, 512, 5, "f32"), (128, 400, 4, "f32"), (256, 200, 4, "f32"), (4, 1000, 12, "f16"),
+            (1, 4096, 4, "f32"), (1, 15000, 3, "f32"))}

@@ -6,20 +6,20 @@ import numpy as np
 import pytest
 
 from palladium_amd import dtypes
-from spread_cases import CASES, CROSSED, LANE_ROWS, OVERWRITTEN
+from spread_cases import CASES, CROSSED, LANE_ROWS, MOMENTS, OVERWRITTEN
 
 pytestmark = pytest.mark.gpu
 
 
 def _run(name, mode):
-    call, args = CASES[name](np.random.default_rng(7), math_mode=mode)
+    call, args = {**CASES, **MOMENTS}[name](np.random.default_rng(7), math_mode=mode)
     print(f"[spread] {name} {mode}", flush=True)
     got, want = call(*args), call.interpret(*args)
     return [got] if isinstance(got, np.ndarray) else got, [want] if isinstance(want, np.ndarray) else want
 
 
 @pytest.mark.parametrize("mode", ["safe", "reproducible"])
-@pytest.mark.parametrize("name", sorted(CASES))
+@pytest.mark.parametrize("name", sorted({**CASES, **MOMENTS}))
 def test_bit_exact_against_the_interpreter(name, mode):
     for g, w in zip(*_run(name, mode)):
         if dtypes.is_bf16(g.dtype):

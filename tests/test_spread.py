@@ -9,12 +9,12 @@ import palladium_amd as pa
 from palladium_amd.emit import emit_hip, launch_geometry
 from palladium_amd.emit.core import plan_of
 from palladium_amd.emit.lanes import LanePlan
-from palladium_amd.emit.spread import MAX_LANES, MAX_SLOTS, SpreadPlan
+from palladium_amd.emit.spread import MAX_LANES, MAX_SLOTS, ORDERED_LDS, SpreadPlan
 from palladium_amd.frontend import jnp, pl
 from palladium_amd.frontend.core import current_builder
 from palladium_amd.ir import ShapedArray
 from palladium_amd.trace import trace
-from spread_cases import CASES, CROSSED, LANE_ROWS, OVERWRITTEN
+from spread_cases import CASES, CROSSED, LANE_ROWS, MOMENTS, OVERWRITTEN
 
 F = np.float32
 
@@ -57,6 +57,15 @@ def test_every_element_has_one_lane(name):
 def test_compiles_without_scratch(name, mode):
     call, args = CASES[name](np.random.default_rng(1), math_mode=mode)
     assert call.explain(*args).resources.scratch_bytes == 0
+
+
+@pytest.mark.parametrize("name", sorted(MOMENTS))
+def test_sums_of_a_kernel_share_their_staging(name):
+    """At most one row array of ORDERED_LDS, and the exchanges of wide teams."""
+    for mode in ("safe", "reproducible"):
+        call, args = MOMENTS[name](np.random.default_rng(1), math_mode=mode)
+        assert isinstance(plan_of(trace(call._staged, *args)), SpreadPlan)
+        assert call.explain(*args).resources.lds_bytes <= ORDERED_LDS + 1024
 
 
 @pytest.mark.parametrize("name, rounds", [("flat_250_bf16", True), ("flat_1250_bf16", True), ("flat_wide_bf16", True),
