@@ -756,16 +756,23 @@ def _tile_plan(p: _Pass, m: int, w: int, programs: int, lane_plan: Any) -> Sprea
     if m < TILE or 4 * across > MAX_SLOTS:
         return None
     down = 2 if 8 * across <= MAX_SLOTS and programs * m >= 2048 * 2 * TILE else 1
-    while -(-m // (TILE * down)) * WAVE > MAX_LANES:
+    while -(-m // (TILE * down)) * WAVE > _lanes_max(programs):
         down *= 2
-    if 4 * across * down > MAX_SLOTS:
-        return None
+        if 4 * across * down > MAX_SLOTS:
+            return None
     return SpreadPlan(m, w, WAVE, 4 * across * down, 1, False, (m, w), (down, across))
+
+
+def _lanes_max(programs: int) -> int:
+    """An instance's lanes: a launch has fewer than 2**31 of them in all."""
+    return min(MAX_LANES, (2**31 - 1) // programs)
 
 
 def _layout(p: _Pass, m: int, w: int, programs: int) -> tuple[int, int, int] | None:
     """(T, R, V) for M rows of W, or None."""
-    limit = MAX_LANES // m
+    limit = _lanes_max(programs) // m
+    if limit < 1:
+        return None
     item = max(p.itemsizes, default=4)
     vmax = max(1, 16 // max(item, 1))
     if not p.reduces:

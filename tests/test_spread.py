@@ -10,7 +10,7 @@ from palladium_amd.emit import emit_hip, launch_geometry
 from palladium_amd.emit.core import plan_of
 from palladium_amd.emit.lanes import LanePlan
 from palladium_amd.emit.spread import MAX_LANES, MAX_SLOTS, ORDERED_LDS, SpreadPlan
-from palladium_amd.frontend import jnp, pl
+from palladium_amd.frontend import jnp, lax, pl
 from palladium_amd.frontend.core import current_builder
 from palladium_amd.ir import ShapedArray
 from palladium_amd.trace import trace
@@ -66,6 +66,47 @@ def test_sums_of_a_kernel_share_their_staging(name):
         call, args = MOMENTS[name](np.random.default_rng(1), math_mode=mode)
         assert isinstance(plan_of(trace(call._staged, *args)), SpreadPlan)
         assert call.explain(*args).resources.lds_bytes <= ORDERED_LDS + 1024
+
+
+def _huge(kind, grid, m, w, k=8):
+    """A kernel over shapes alone."""
+    def loop(x_ref, o_ref):
+        o_ref[...] = lax.fori_loop(0, 5, lambda _, y: y * 0.5 + 1.0, x_ref[...])
+
+    def softmax(x_ref, o_ref):
+        e = jnp.exp(x_ref[...] - jnp.max(x_ref[...], axis=-1, keepdims=True))
+        o_ref[...] = e / jnp.sum(e, axis=-1, keepdims=True)
+
+    def dense(x_ref, w_ref, o_ref):
+        o_ref[...] = jnp.dot(x_ref[...], w_ref[...])
+
+    def block(m, w):
+        return pl.BlockSpec((m, w), lambda i: (i, 0))
+
+    specs, shapes = [block(m, w)], [(grid * m, w)]
+    if kind == "dense":
+        specs, shapes = [block(m, k), pl.BlockSpec((k, w), lambda i: (0, 0))], [(grid * m, k), (k, w)]
+    kernel = {"loop": loop, "softmax": softmax, "dense": dense}[kind]
+    call = pa.hip_call(kernel, grid=(grid,), in_specs=specs, out_specs=block(m, w),
+                       out_shape=pl.ShapeDtypeStruct((grid * m, w), F))
+    return trace(call._staged, *[pl.ShapeDtypeStruct(s, F) for s in shapes])
+
+
+@pytest.mark.parametrize("kind, m, w", [("loop", 1, 100), ("loop", 1, 1000), ("loop", 4, 25), ("softmax", 1, 33),
+                                        ("softmax", 1, 1000), ("softmax", 4, 100), ("dense", 32, 20), ("dense", 48, 64)])
+def test_large_grids_stay_below_the_lane_limit(kind, m, w):
+    """A launch has fewer than 2**31 lanes: with more instances each takes
+    fewer, or one."""
+    free = plan_of(_huge(kind, 1000, m, w))
+    assert isinstance(free, SpreadPlan)
+    edge = (2**31 - 1) // plan_of(_huge(kind, 200_000, m, w)).lanes
+    for grid in (edge, edge + 1, 2 * edge, 2**31 // 3):
+        spec = _huge(kind, grid, m, w)
+        geo, plan = launch_geometry(spec), plan_of(spec)
+        assert geo.lanes * grid < 2**31 and (plan is None) == (geo.lanes == 1)
+        if grid == edge:
+            assert isinstance(plan, SpreadPlan)
+        emit_hip(spec, math_mode="fast")
 
 
 @pytest.mark.parametrize("name, rounds", [("flat_250_bf16", True), ("flat_1250_bf16", True), ("flat_wide_bf16", True),
