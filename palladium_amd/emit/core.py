@@ -462,7 +462,8 @@ def plan_of(spec: KernelSpec) -> Any:
     memo = vars(spec)
     if "_spread_plan" not in memo:
         memo["_spread_plan"] = spread_transform(spec, lanes)
-    return memo["_spread_plan"] or lanes
+    plan = memo["_spread_plan"]
+    return plan if plan is not None and own_rules(plan) else lanes
 
 
 def _may_regroup(math_mode: Any) -> bool:

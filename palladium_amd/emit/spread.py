@@ -822,11 +822,14 @@ def staging(env: Environment) -> list[str]:
     return [f"    __shared__ __attribute__((aligned(16))) unsigned char {STAGING}[{n}];"] if n else []
 
 
-def own_rules() -> bool:
-    """Whether the rules this lowering stands in for are the built-in ones
-    (a user's own rule for an access or a reduction keeps its say)."""
+def own_rules(plan: SpreadPlan | None = None) -> bool:
+    """Whether the rules this lowering stands in for are the built-in ones (a
+    user's own rule for an access, a reduction or, in tiles, a product keeps
+    its say)."""
     from palladium_amd.emit.core import RULES
 
+    if plan is not None and plan.tile:
+        return RULES["dot_general"].__module__ == "palladium_amd.emit.rules"
     return all(RULES[n].__module__ == "palladium_amd.emit.rules"
                for n in ("get", "swap", "iota", "broadcast_in_dim", "reshape", "squeeze", "expand_dims", *_REDUCE))
 

@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 import palladium_amd as pa
-from palladium_amd.emit import emit_hip, launch_geometry
+from palladium_amd.emit import RULES, emit_hip, launch_geometry
 from palladium_amd.emit.core import plan_of
 from palladium_amd.emit.lanes import LanePlan
 from palladium_amd.emit.spread import MAX_LANES, MAX_SLOTS, ORDERED_LDS, SpreadPlan
@@ -211,6 +211,22 @@ def test_disjoint_stores_of_one_output_are_spread():
     call = pa.hip_call(kernel, grid=(3,), in_specs=[pl.BlockSpec((4, 40), lambda i: (i, 0))],
                        out_specs=pl.BlockSpec((4, 3), lambda i: (i, 0)), out_shape=pl.ShapeDtypeStruct((12, 3), F))
     assert isinstance(plan_of(trace(call._staged, np.zeros((12, 40), F))), SpreadPlan)
+
+
+@pytest.mark.parametrize("name, primitive", [("dense_64x21x17_f32", "dot_general"), ("dense_33x7x33_f16", "dot_general"),
+                                             ("rows_8x128_f32", "reduce_max"), ("flat_1000_u32", "get")])
+def test_a_rule_of_ones_own_keeps_its_say(name, primitive, monkeypatch):
+    built_in = RULES[primitive]
+
+    def own(env, cursor, eqn):
+        cursor.emit("// the user's rule")
+        built_in(env, cursor, eqn)
+
+    spec = _spec(name)
+    assert isinstance(plan_of(spec), SpreadPlan)
+    monkeypatch.setitem(RULES, primitive, own)
+    assert "// the user's rule" in emit_hip(spec, math_mode="fast")
+    assert not isinstance(plan_of(spec), SpreadPlan)
 
 
 def test_small_blocks_and_plain_gridless_calls_keep_one_lane():
