@@ -26,7 +26,7 @@ from typing import Any
 from palladium_amd.dtypes import name as _dtype_name
 
 from palladium_amd.diagnostics import KernelDiagnostics, explain_spec, log_compile
-from palladium_amd.emit import emit_hip, launch_geometry
+from palladium_amd.emit import LaunchGeometry, emit_hip, launch_geometry
 from palladium_amd.runtime import REPRODUCIBLE_ORDINAL, MathMode, math_mode_ordinal
 from palladium_amd.trace import KernelSpec, trace
 
@@ -106,13 +106,18 @@ class FfiCallable:
             self.interpret = functools.partial(interpret_call, self._staged, math_mode=self._math_mode)
         self._vmap_method = vmap_method
         self._threadgroup = threadgroup
-        self._cache: dict[tuple, tuple[KernelSpec, str]] = {}
+        self._cache: dict[tuple, tuple[KernelSpec, str, LaunchGeometry]] = {}
         self._lock = threading.Lock()
 
     def explain(self, *args: Any, compile: bool = True) -> KernelDiagnostics:
         return explain_spec(trace(self._staged, *args), self._threadgroup, self._math_mode, compile=compile)
 
     def spec_and_source(self, args: tuple) -> tuple[KernelSpec, str]:
+        return self._entry(args)[:2]
+
+    def _entry(self, args: tuple) -> tuple[KernelSpec, str, LaunchGeometry]:
+        """The spec, its source and the launch that source was emitted for
+        (rules registered later change neither)."""
         key = tuple((tuple(a.shape), _dtype_name(a.dtype)) for a in args)
         entry = self._cache.get(key)
         if entry is None:
@@ -126,17 +131,15 @@ class FfiCallable:
                     spec = trace(self._staged, *args)
                     check_block_bounds(spec)
                     log_compile(spec, self._threadgroup, self._math_mode)
-                    entry = (spec, emit_hip(spec, block=_block_of(self._threadgroup), math_mode=self._math_mode,
-                                     tile=_tile_of(self._threadgroup)))
+                    block = _block_of(self._threadgroup)
+                    entry = (spec, emit_hip(spec, block=block, math_mode=self._math_mode,
+                                            tile=_tile_of(self._threadgroup)), launch_geometry(spec, block))
                     self._cache[key] = entry
         return entry
 
     def ffi_attributes(self, args: tuple) -> dict[str, Any]:
         """The attribute dict handed to the native handler for these shapes."""
-        from palladium_amd.dispatch import _block_of
-
-        spec, src = self.spec_and_source(args)
-        geo = launch_geometry(spec, _block_of(self._threadgroup))
+        spec, src, geo = self._entry(args)
         grid = tuple(spec.grid) + (1, 1, 1)
         if len(spec.grid) > 3:
             grid = (spec.num_programs, 1, 1)

@@ -163,6 +163,21 @@ def test_ffi_attributes_carry_lanes_of_a_lane_parallel_kernel():
     assert (attrs["grid_x"], attrs["block_x"], attrs["lanes"]) == (8, 128, 128)
 
 
+def test_ffi_launch_is_the_one_its_source_was_emitted_for(monkeypatch):
+    """Also after a rule is registered that another lowering would be for."""
+    from palladium_amd.emit import RULES
+
+    s = pl.BlockSpec((1000,), lambda i: (i,))
+    fn = pa.hip_call_jit(lambda x_ref, o_ref: o_ref.__setitem__(..., x_ref[...] * 2.0), grid=(3,), in_specs=[s], out_specs=s,
+                         out_shape=pl.ShapeDtypeStruct((3000,), np.float32))
+    x = np.zeros(3000, np.float32)
+    before = fn.ffi_attributes((x,))
+    assert before["lanes"] > 1 and f"block={before['block_x']} " in before["hip_source"]
+    built_in = RULES["get"]
+    monkeypatch.setitem(RULES, "get", lambda env, cursor, eqn: built_in(env, cursor, eqn))
+    assert fn.ffi_attributes((x,)) == before
+
+
 def test_math_mode_values():
     assert pa.MathMode("safe").ordinal == 0 and pa.MathMode.FAST.ordinal == 2
     with pytest.raises(ValueError):
