@@ -114,6 +114,12 @@ def row_stride(width: int) -> int:
     (four elements a read) whose starts fall on different banks."""
     return -(-width // 4) * 4 + 4
 
+
+def staged_rows(width: int, team: int, workgroup: int) -> int:
+    """Bytes of the rows that a workgroup's teams stage."""
+    return max(1, workgroup // team) * row_stride(width) * 4
+
+
 # Element-wise primitives the rewrites of `optimize` add to the traced ones.
 _POINTWISE = _ELEMENTWISE | {"fma", "alignbit", "pow_log", "pow_with_log"}
 _CALLS = {"pjit", "jit", "closed_call", "core_call", "custom_jvp_call", "custom_vjp_call"}
@@ -155,11 +161,14 @@ class SpreadPlan:
 
     def workgroup(self, block: int | None, default: int) -> int:
         """A reducing team wider than a wavefront is one workgroup (its lanes
-        meet at barriers); narrower ones share the default workgroup (ordered
-        sums stage its rows in LDS)."""
-        if self.reduces:
-            return self.team if self.team > WAVE else default
-        return block or default
+        meet at barriers), whatever was asked for; narrower ones share the
+        workgroup asked for as long as the rows of an ordered sum fit (the
+        default's do)."""
+        if not self.reduces:
+            return block or default
+        if self.team > WAVE:
+            return self.team
+        return block if block and staged_rows(self.width, self.team, block) <= ORDERED_LDS else default
 
 
 Status = Any  # None (plain) or a tuple of 'm' / 'w' / 'u', one per dim
@@ -876,7 +885,7 @@ def spread_transform(spec: KernelSpec, lane_plan: Any = None) -> SpreadPlan | No
         if lane_plan is not None and m == 1 and vec == 1:
             continue
         if p.reduces:
-            if max(1, DEFAULT_WORKGROUP // team) * row_stride(width) * 4 > ORDERED_LDS:
+            if staged_rows(width, team, DEFAULT_WORKGROUP) > ORDERED_LDS:
                 continue
         return SpreadPlan(rows, width, team, slots, vec, p.reduces, (m, w),
                           rounded=lane_plan is None and m * w >= MIN_ROUNDED)

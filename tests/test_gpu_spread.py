@@ -83,3 +83,14 @@ def test_lanes_of_an_instance_keep_its_order(name, mode):
     got, want = call(*args), call.interpret(*args)
     for g, w in zip(*((v,) if isinstance(v, np.ndarray) else v for v in (got, want))):
         np.testing.assert_array_equal(g, w)
+
+
+@pytest.mark.parametrize("block", [64, 512, 1024])
+@pytest.mark.parametrize("name", ["rows_4x17_f32", "rows_8x128_f32", "rows_64x40_f32", "dense_64x21x17_f32"])
+def test_results_do_not_depend_on_the_workgroup(name, block):
+    for mode in ("safe", "fast"):
+        call, args = CASES[name](np.random.default_rng(7), math_mode=mode, threadgroup=block)
+        default, _ = CASES[name](np.random.default_rng(7), math_mode=mode)
+        print(f"[spread] {name} {block} {mode}", flush=True)
+        for g, w in zip(*((v,) if isinstance(v, np.ndarray) else v for v in (call(*args), default(*args)))):
+            np.testing.assert_array_equal(g, w)

@@ -229,6 +229,18 @@ def test_a_rule_of_ones_own_keeps_its_say(name, primitive, monkeypatch):
     assert not isinstance(plan_of(spec), SpreadPlan)
 
 
+@pytest.mark.parametrize("name, block, taken", [
+    *((n, b, b) for n in ("rows_4x17_f32", "rows_8x128_f32", "rows_64x40_f32", "flat_1250_bf16", "dense_64x21x17_f32")
+      for b in (64, 512, 1024)),
+    ("rows_1x1000_f32", 64, 256), ("rows_1x1000_f32", 1024, 256),  # a team of 256 is a workgroup
+    ("moments_64x900_3_f32", 1024, 256)])  # 230 KB of rows
+def test_the_workgroup_asked_for(name, block, taken):
+    call, args = {**CASES, **MOMENTS}[name](np.random.default_rng(1), threadgroup=block, math_mode="safe")
+    diag = call.explain(*args)
+    assert diag.block == taken and diag.blocks * diag.block >= trace(call._staged, *args).num_programs * diag.lanes
+    assert diag.resources.lds_bytes <= ORDERED_LDS + 1024
+
+
 def test_small_blocks_and_plain_gridless_calls_keep_one_lane():
     def double(x_ref, o_ref):
         o_ref[...] = x_ref[...] * 2.0
