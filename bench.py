@@ -600,7 +600,7 @@ def bench_gs(steps: int, warmup: int, cpu: bool) -> dict:
     ms = gpu_s * 1e3 / n_steps
     achieved = GS_BYTES_PER_CELL_STEP * cells / (ms / 1e3)
     res = _base("Gray-Scott cell-steps/s (4096^2, 2,000 steps, fp32)", cells / (ms / 1e3), "cell-steps/s",
-                n_steps, 10, ms, {"workload": "Gray-Scott 4096x4096, 2000 steps as one HIP graph, config 4",
+                n_steps, 10, ms, {"workload": f"Gray-Scott 4096x4096, 2000 steps as one {'HIP graph' if graph else 'batch'}, config 4",
                                   "size": cfg.size, "math_mode": "fast"})
     res["roofline"] = {"bound": "hbm", "achieved": achieved / 1e9, "peak": HBM_PEAK / 1e9, "unit": "GB/s",
                        "frac": achieved / HBM_PEAK, "traffic": GS_MEASURED_TRAFFIC_BYTES, "bytes_per_cell_step": GS_BYTES_PER_CELL_STEP,
@@ -708,8 +708,8 @@ def bench_gs_fused(steps: int, warmup: int, cpu: bool) -> dict:
     hbm = pass_bytes * passes / (gpu_s)
     res = _base("Gray-Scott cell-steps/s (4096^2, 2,000 steps, fp32), temporal blocking", cells / (ms / 1e3),
                 "cell-steps/s", n_steps, 2 * k, ms,
-                {"workload": f"Gray-Scott 4096x4096, {n_steps} steps in {passes} passes ({k} steps each) as one HIP "
-                             f"graph, config 4; {fused.describe()}", "size": cfg.size, "math_mode": "fast",
+                {"workload": f"Gray-Scott 4096x4096, {n_steps} steps in {passes} passes ({k} steps each) as one "
+                             f"{'HIP graph' if graph else 'batch'}, config 4; {fused.describe()}", "size": cfg.size, "math_mode": "fast",
                  "kernel": kind, "steps_per_pass": k})
     traffic = {"lds": GSF_MEASURED_TRAFFIC_BYTES, "regs": GSR_MEASURED_TRAFFIC_BYTES}[kind]
     res["roofline"] = {"bound": "issue", "achieved": hbm / 1e9, "peak": HBM_PEAK / 1e9, "unit": "GB/s",
@@ -796,8 +796,8 @@ def bench_gs_geometry(steps: int, warmup: int, cpu: bool) -> dict:
     for rows, group, k, cols in GS_GEOMETRIES:
         f = stencil.RegisterGrayScott(n, k=k, rows=rows, group=group, cols=cols)
         stencil.gray_scott_fused_run(f, u0, v0, 2 * k)
-        stencil.gray_scott_fused_run(f, u0, v0, n_steps)
-        best = min(stencil.gray_scott_fused_run(f, u0, v0, n_steps)[2] for _ in range(3))
+        stencil.gray_scott_fused_run(f, u0, v0, n_steps, graph=True)
+        best = min(stencil.gray_scott_fused_run(f, u0, v0, n_steps, graph=True)[2] for _ in range(3))
         r = diagnostics.code_object_resources(rt.compile_code_object(f.source(k), "gray_scott_regs", "fast"),
                                               "gray_scott_regs")
         waves = stencil.register_geometry(n, k, rows, cols)[0]

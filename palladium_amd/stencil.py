@@ -493,10 +493,10 @@ class RegisterGrayScott:
         return [self.k] * (steps // self.k) + [1] * (steps % self.k)
 
 
-def gray_scott_fused_run(fused: FusedGrayScott | RegisterGrayScott, u0: np.ndarray, v0: np.ndarray, steps: int, graph: bool = True):
+def gray_scott_fused_run(fused: FusedGrayScott | RegisterGrayScott, u0: np.ndarray, v0: np.ndarray, steps: int, graph: bool = False):
     """`steps` Gray-Scott steps in passes of `fused.k`, ping-ponging two
-    buffer pairs, queued as one batch, which runs once and so is submitted
-    launch by launch whatever `graph` says (`workloads.gray_scott_run`).
+    buffer pairs, queued as one batch (one HIP graph when `graph`, which a
+    batch that runs once does not pay back: `workloads.gray_scott_run`).
     Returns (u, v, device seconds)."""
     if u0.shape != (fused.n, fused.n) or v0.shape != u0.shape:
         raise ValueError(f"fields must be {fused.n}x{fused.n}")
@@ -515,7 +515,7 @@ def gray_scott_fused_run(fused: FusedGrayScott | RegisterGrayScott, u0: np.ndarr
     passes = fused.launches(steps)
     for i, kk in enumerate(passes):
         batch.add(fused._kernels[kk], fused.blocks_for(kk), WORKGROUP, ptrs[i % 2])
-    batch.commit()
+    batch.commit(graph=graph)
     batch.wait()
     u, v = bufs[len(passes) % 2]
     return u.to_numpy(stream), v.to_numpy(stream), batch.gpu_time

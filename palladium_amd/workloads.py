@@ -535,13 +535,13 @@ def gray_scott_initial(size: int, seed: int = GS_CFG.seed) -> tuple[np.ndarray, 
 GS_BYTES_PER_CELL_STEP = 16
 
 
-def gray_scott_run(call, u0: np.ndarray, v0: np.ndarray, steps: int, graph: bool = True):
+def gray_scott_run(call, u0: np.ndarray, v0: np.ndarray, steps: int, graph: bool = False):
     """Run `steps` Gray-Scott steps on the GPU, ping-ponging two buffer pairs,
-    all launches queued as one batch; the multi-launch driver of
-    `examples/04_reaction_diffusion.py:77-109`. The batch runs once, so it is
-    submitted launch by launch whatever `graph` says: recording 200 launches
-    of a 500 x 500 step into a HIP graph takes 0.40 ms before the first can
-    start and running it 0.50, submitting them 0.50 in all.
+    all launches queued as one batch (one HIP graph when `graph`); the
+    multi-launch driver of `examples/04_reaction_diffusion.py:77-109`. The
+    batch runs once, so a graph does not pay: recording 200 launches of a
+    500 x 500 step takes 0.40 ms before the first can start and running it
+    0.50, submitting them 0.50 in all.
     Returns (u, v, device seconds)."""
     from palladium_amd import runtime as rt
 
@@ -555,7 +555,7 @@ def gray_scott_run(call, u0: np.ndarray, v0: np.ndarray, steps: int, graph: bool
     batch = rt.Batch(stream=bound.stream)
     for step in range(steps):
         batch.add(bound.kernel, geo.blocks, geo.block, ptrs[step % 2])
-    batch.commit()
+    batch.commit(graph=graph)
     batch.wait()
     u, v = bufs[steps % 2]
     return u.to_numpy(bound.stream), v.to_numpy(bound.stream), batch.gpu_time

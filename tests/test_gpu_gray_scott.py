@@ -59,7 +59,7 @@ def test_full_config4_safe_bit_exact():
     equal to the oracle bit for bit."""
     size, steps = GS_CFG.size, GS_CFG.steps
     u0, v0 = gray_scott_initial(size)
-    u, v, _ = gray_scott_run(gray_scott_call(size=size, math_mode="safe"), u0, v0, steps)
+    u, v, _ = gray_scott_run(gray_scott_call(size=size, math_mode="safe"), u0, v0, steps, graph=True)
     wu, wv = oracle.gray_scott(u0, v0, GS_CFG, steps)
     np.testing.assert_array_equal(u, wu)
     np.testing.assert_array_equal(v, wv)

@@ -88,3 +88,14 @@ def test_uniform_state_is_a_fixed_point(kind):
     u, v, _ = stencil.gray_scott_fused_run(KINDS[kind](n), u0, v0, 20)
     np.testing.assert_array_equal(u, u0)
     np.testing.assert_array_equal(v, v0)
+
+
+@pytest.mark.parametrize("kind", sorted(KINDS))
+def test_passes_as_one_graph_equal_the_oracle(kind):
+    n, steps = 256, 13
+    u0, v0 = gray_scott_initial(n)
+    print(f"[stencil] {kind} graph", flush=True)
+    u, v, _ = stencil.gray_scott_fused_run(KINDS[kind](n, math_mode="safe"), u0, v0, steps, graph=True)
+    wu, wv = oracle.gray_scott(u0, v0, GS_CFG, steps)
+    np.testing.assert_array_equal(u, wu)
+    np.testing.assert_array_equal(v, wv)

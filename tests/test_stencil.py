@@ -215,3 +215,52 @@ def test_runner_checks_its_arguments_before_touching_a_device():
         stencil.gray_scott_fused_run(f, u0, u0, -1)
     u, v, t = stencil.gray_scott_fused_run(f, u0, 2 * u0, 0)
     assert t == 0.0 and np.array_equal(u, u0) and np.array_equal(v, 2 * u0) and u is not u0
+
+
+@pytest.mark.parametrize("graph", [None, False, True])
+def test_drivers_record_a_graph_when_asked(monkeypatch, graph):
+    """Both drivers hand `graph` to the batch (no graph unless asked)."""
+    from palladium_amd import workloads
+
+    asked = []
+
+    class Buffer:
+        ptr = 0
+
+        @classmethod
+        def from_numpy(cls, a):
+            return cls()
+
+        @classmethod
+        def empty(cls, shape, dtype):
+            return cls()
+
+        def to_numpy(self, stream):
+            return None
+
+    class Batch:
+        gpu_time = 0.0
+
+        def __init__(self, stream=None):
+            pass
+
+        def add(self, *a):
+            pass
+
+        def commit(self, graph=False):
+            asked.append(graph)
+
+        def wait(self):
+            pass
+
+    monkeypatch.setattr(rt, "Buffer", Buffer)
+    monkeypatch.setattr(rt, "Batch", Batch)
+    monkeypatch.setattr(rt, "Stream", lambda: None)
+    kw = {} if graph is None else {"graph": graph}
+    u0, v0 = gray_scott_initial(128)
+    stencil.gray_scott_fused_run(stencil.RegisterGrayScott(128), u0, v0, 7, **kw)
+    call = workloads.gray_scott_call(size=128)
+    bound = call.bound(u0, v0)
+    bound._stream.append(None)
+    workloads.gray_scott_run(call, u0, v0, 3, **kw)
+    assert asked == [bool(graph)] * 2
