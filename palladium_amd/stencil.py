@@ -456,14 +456,13 @@ def _consts(cfg: Any) -> tuple:
 @dataclasses.dataclass
 class RegisterGrayScott:
     """A compiled K-step register pass (`register_source`) and a one-step
-    pass of the same code for step counts K does not divide. `rows` other
-    than the default is the height of the strips as given; at the default it
-    is the tallest that `strip_height` may choose. Results do not depend on
-    it."""
+    pass of the same code for step counts K does not divide. `rows` is the
+    height of the strips; None takes `strip_height`'s choice for the grid.
+    Results do not depend on it."""
 
     n: int
     k: int = 6
-    rows: int = 64
+    rows: int | None = None
     group: int = 4
     math_mode: Any = "fast"
     cfg: Any = None
@@ -471,9 +470,10 @@ class RegisterGrayScott:
 
     def __post_init__(self) -> None:
         consts = _consts(self.cfg)
-        chosen = self.rows == DEFAULT_ROWS and self.cols == 1 and self.rows + 2 * self.k <= self.n
-        height = strip_height(self.n, self.k, self.rows, self.group) if chosen else self.rows
-        self._rows = {kk: height for kk in {self.k, 1}}
+        if self.rows is None:
+            adapts = self.cols == 1 and DEFAULT_ROWS + 2 * self.k <= self.n
+            self.rows = strip_height(self.n, self.k, group=self.group) if adapts else DEFAULT_ROWS
+        self._rows = {kk: self.rows for kk in {self.k, 1}}
         self._src = {kk: register_source(self.n, kk, r, *consts, group=self.group, cols=self.cols)
                      for kk, r in self._rows.items()}
         self._kernels = {kk: rt.Kernel(src, "gray_scott_regs", self.math_mode) for kk, src in self._src.items()}

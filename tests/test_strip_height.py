@@ -28,6 +28,7 @@ def test_default_adapts_and_explicit_heights_stay():
     assert stencil.RegisterGrayScott(200)._rows == {6: 2, 1: 2}
     assert stencil.RegisterGrayScott(4096)._rows == {6: 64, 1: 64}
     assert stencil.RegisterGrayScott(512, rows=40)._rows == {6: 40, 1: 40}
+    assert stencil.RegisterGrayScott(512, rows=64)._rows == {6: 64, 1: 64}
     assert stencil.RegisterGrayScott(512, cols=2)._rows == {6: 64, 1: 64}
     with pytest.raises(ValueError, match="too small"):
         stencil.RegisterGrayScott(75)
