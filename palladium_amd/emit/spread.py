@@ -146,7 +146,6 @@ class SpreadPlan:
     reduces: bool
     block: tuple[int, int]  # the block as traced (rows and width before flattening)
     tile: tuple[int, int] | None = None  # dots: 16 x 16 tiles down and across a wavefront's part
-
     rounded: bool = False  # bfloat16 operations round one by one in every mode (`MIN_ROUNDED`)
 
     @property
@@ -769,7 +768,11 @@ def _tile_plan(p: _Pass, m: int, w: int, programs: int, lane_plan: Any) -> Sprea
         down *= 2
         if 4 * across * down > MAX_SLOTS:
             return None
-    return SpreadPlan(m, w, WAVE, 4 * across * down, 1, False, (m, w), (down, across))
+    return SpreadPlan(m, w, WAVE, 4 * across * down, 1, False, (m, w), (down, across), _rounds(m, w, lane_plan))
+
+
+def _rounds(m: int, w: int, lane_plan: Any) -> bool:
+    return lane_plan is None and m * w >= MIN_ROUNDED
 
 
 def _lanes_max(programs: int) -> int:
@@ -887,8 +890,7 @@ def spread_transform(spec: KernelSpec, lane_plan: Any = None) -> SpreadPlan | No
         if p.reduces:
             if staged_rows(width, team, DEFAULT_WORKGROUP) > ORDERED_LDS:
                 continue
-        return SpreadPlan(rows, width, team, slots, vec, p.reduces, (m, w),
-                          rounded=lane_plan is None and m * w >= MIN_ROUNDED)
+        return SpreadPlan(rows, width, team, slots, vec, p.reduces, (m, w), rounded=_rounds(m, w, lane_plan))
     return None
 
 

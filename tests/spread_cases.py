@@ -214,7 +214,7 @@ CASES = {
        ((128, 64, 32, "f32"), (64, 21, 17, "f32"), (100, 33, 3, "f32"), (16, 16, 16, "f32"), (1024, 16, 48, "f32"),
         (250, 40, 64, "bf16"), (64, 32, 30, "bf16"), (128, 96, 16, "f16"), (33, 7, 33, "f16"), (256, 128, 64, "f32"),
         (64, 15, 40, "f16"), (64, 3, 18, "bf16"), (64, 1, 20, "f16"), (64, 2, 24, "f32"), (128, 50, 20, "f32"),
-        (64, 84, 24, "f16"), (64, 8, 17, "bf16"))},
+        (64, 84, 24, "f16"), (64, 8, 17, "bf16"), (33, 1, 40, "bf16"))},
     "dense_64x24x20_transposed_f32": dense(64, 24, 20, "f32", transposed=True),
     "dense_64x40x20_transposed_bf16": dense(64, 40, 20, "bf16", transposed=True),
     "dense_wide_f32": dense(128, 24, 32, "f32", grid=600),

@@ -50,7 +50,7 @@ def test_fast_close_to_the_interpreter(name):
 
 
 @pytest.mark.parametrize("mode", ["fast", "relaxed"])
-@pytest.mark.parametrize("name", ["flat_250_bf16", "flat_1250_bf16", "flat_wide_bf16"])
+@pytest.mark.parametrize("name", ["flat_250_bf16", "flat_1250_bf16", "flat_wide_bf16", "dense_33x1x40_bf16"])
 def test_bfloat16_operations_round_one_by_one(name, mode):
     """Sums and products rounded each: the interpreter's bits. (No operation
     here leaves the exactly rounded ones, and no value is subnormal.)"""
