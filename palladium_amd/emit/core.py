@@ -105,6 +105,8 @@ class CVal:
         operand refs and views of them.
     readonly : bool
         True for input refs and views of them.
+    steps : tuple of (size, stride), or None
+        Dims of a view whose elements do not lie side by side (a column).
     """
 
     expr: str
@@ -112,6 +114,7 @@ class CVal:
     ctype: str
     space: str = "local"
     readonly: bool = False
+    steps: tuple[tuple[int, int], ...] | None = None
 
     @property
     def size(self) -> int:
@@ -127,7 +130,14 @@ class CVal:
         size-1 locals."""
         if self.scalar:
             return self.expr
-        return f"{self.expr}[{index}]"
+        if self.steps is None:
+            return f"{self.expr}[{index}]"
+        terms, inner = [], 1
+        for k, (n, stride) in reversed(list(enumerate(self.steps))):
+            place = f"({index})" if inner == 1 else f"({index}) / {inner}"
+            terms.append(f"{place} % {n} * {stride}" if k else f"{place} * {stride}")
+            inner *= n
+        return f"{self.expr}[{' + '.join(reversed(terms))}]"
 
 
 class Cursor:
@@ -342,8 +352,10 @@ def ref_view(env: Environment, ref: CVal, indexer: NDIndexer) -> CVal:
     """Pointer offset + kept shape for an indexed ref access.
 
     A Slice keeps its dim, any other index squeezes it into the offset.
-    Only the first kept dim may be partial (contiguous access), as in the
-    reference (`src/palladium/emit/core.py:469-545`).
+    Only the first kept dim may be partial, as in the reference
+    (`src/palladium/emit/core.py:469-545`). An index after a kept dim (a
+    column, `x_ref[:, j]`) leaves gaps between the view's elements: its
+    `steps` tell them, and `at` counts them in.
     """
     strides = element_strides(tuple(indexer.shape))
     terms: list[str] = []
@@ -370,7 +382,9 @@ def ref_view(env: Environment, ref: CVal, indexer: NDIndexer) -> CVal:
     shape = tuple(size for _, size in kept)
     base = ref.expr
     expr = f"({base} + {offset})" if offset != "0" else base
-    return CVal(expr, shape if shape else (1,), ref.ctype, "global", ref.readonly)
+    steps = tuple((size, strides[d]) for d, size in kept if size != 1)
+    side_by_side = all(s == math.prod(n for n, _ in steps[k + 1:]) for k, (_, s) in enumerate(steps))
+    return CVal(expr, shape if shape else (1,), ref.ctype, "global", ref.readonly, None if side_by_side else steps)
 
 
 def _emit_block_offset(env: Environment, cursor: Cursor, spec: KernelSpec, info: BlockInfo, pid_vals: list[CVal]) -> str:

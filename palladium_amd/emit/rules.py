@@ -331,7 +331,7 @@ def _rule_get(env: Environment, cursor: Cursor, eqn: JaxprEqn) -> None:
     if size == 1:
         declare(env, cursor, out, init=view.at("0"))
         return
-    if view.readonly and size > REGISTER_BLOCK_LIMIT:
+    if view.readonly and size > REGISTER_BLOCK_LIMIT and view.steps is None:
         env.bind(out, dataclasses.replace(view, shape=out_shape))
         return
     dst = declare(env, cursor, out)

@@ -9,6 +9,7 @@ from palladium_amd.emit import emit_hip, rule
 from palladium_amd.errors import EmitError, UnsupportedPrimitiveError
 from palladium_amd.frontend import jnp, lax, pl, random
 from palladium_amd.interpret import interpret_call
+from palladium_amd.ir import Literal, ShapedArray
 from palladium_amd.trace import trace
 
 
@@ -273,3 +274,27 @@ def test_empty_grid_is_a_clear_error_and_interprets_to_empty():
     assert np.asarray(f.interpret(x)).shape == (0,)
     with pytest.raises(EmitError, match="no program instances"):
         f.explain(x, compile=False)
+
+
+@pytest.mark.parametrize("shape, index", [
+    ((4, 6), (slice(None), 5)), ((4, 6), (2, slice(None))), ((3, 4, 5), (slice(None), 2, slice(None))),
+    ((3, 4, 5), (slice(None), slice(None), 4)), ((3, 4, 5), (slice(1, 3), 0, slice(None))), ((3, 4, 5), (2, slice(None), 3)),
+    ((3, 1, 5), (slice(None), 0, slice(None))), ((3, 4, 1), (slice(None), slice(None), 0)), ((1, 6), (slice(None), 3)),
+    ((2, 3, 4, 5), (slice(None), 1, slice(None), 2))])
+def test_views_step_over_what_they_leave_out(shape, index):
+    """The element a view's flat index reaches is NumPy's, whatever dims the
+    index leaves out."""
+    from palladium_amd.emit.core import CVal, Environment, ref_view
+    from palladium_amd.ir import NDIndexer, Slice
+
+    flat = np.arange(np.prod(shape)).reshape(shape)
+    ixs = tuple(Slice(ix.start or 0, len(range(*ix.indices(n))), 1) if isinstance(ix, slice) else Literal(ix, ShapedArray((), np.int32))
+                for ix, n in zip(index, shape))
+    view = ref_view(Environment("int"), CVal("r", shape, "float", "global"), NDIndexer(ixs, shape))
+    want = flat[index].reshape(-1)
+    base = int(eval(view.expr.replace("(int)", "").replace("r", "0")))
+    name = view.expr.replace("[", "")
+    for i, w in enumerate(want):
+        at = view.at(str(i))
+        assert at.startswith(name + "[") and base + eval(at[len(name) + 1:-1].replace("/", "//")) == w
+    assert (view.steps is None) == bool((np.diff(want) == 1).all())

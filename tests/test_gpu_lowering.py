@@ -272,3 +272,45 @@ def test_divergent_while_per_lane():
     f = pa.hip_call(kernel, grid=(300,), out_specs=pl.BlockSpec((1,), lambda i: (i,)),
                     out_shape=SDS((300,), F), math_mode="safe")
     _both(f)
+
+
+@pytest.mark.parametrize("m, w", [(3, 5), (7, 2), (2, 7), (20, 3)])
+def test_columns_of_a_block(m, w, rng):
+    """One lane per instance: columns read, swapped and stored, also with
+    an index that is only known at run time."""
+    def kernel(x_ref, o_ref, p_ref):
+        o_ref[...] = x_ref[...]
+        o_ref[:, 0] = x_ref[:, w - 1] * 2.0
+        o_ref[:, w - 1] = x_ref[:, 0] + 1.0
+
+        def body(j, c):
+            p_ref[:, j] = x_ref[:, w - 1 - j] + c
+            return c + 1.0
+
+        lax.fori_loop(0, w, body, jnp.float32(0.0))
+        p_ref[m - 1, :] = o_ref[0, :]
+
+    blk = pl.BlockSpec((m, w), lambda i: (i, 0))
+    f = pa.hip_call(kernel, grid=(5,), in_specs=[blk], out_specs=(blk, blk),
+                    out_shape=(SDS((5 * m, w), F), SDS((5 * m, w), F)), math_mode="safe")
+    x = rng.standard_normal((5 * m, w), dtype=F)
+    o, p = _both(f, x)
+    np.testing.assert_array_equal(o[:, 0], x[:, w - 1] * F(2.0))
+    want = x[:, ::-1] + np.arange(w, dtype=F)
+    want[m - 1::m] = o[0::m]
+    np.testing.assert_array_equal(p, want)
+
+
+def test_views_of_three_dims(rng):
+    def kernel(x_ref, o_ref):
+        o_ref[:, 0, :] = x_ref[:, 2, :] * 2.0
+        o_ref[:, 1, :] = x_ref[:, 1, :]
+        o_ref[:, 2, :] = x_ref[:, 0, :] + o_ref[:, 1, :]
+        o_ref[1:3, 2, :] = x_ref[0:2, 0, :]
+        o_ref[0, 2, :] = x_ref[:, 1, 3]
+        o_ref[3, 2, :] = x_ref[:, 1, 3]
+
+    blk = pl.BlockSpec((4, 3, 4), lambda i: (i, 0, 0))
+    f = pa.hip_call(kernel, grid=(2,), in_specs=[blk], out_specs=blk, out_shape=SDS((8, 3, 4), F), math_mode="safe")
+    x = rng.standard_normal((8, 3, 4), dtype=F)
+    _both(f, x)
