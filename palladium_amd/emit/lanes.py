@@ -161,6 +161,10 @@ class _Pass:
         self.access(e.invars[0], "one=" if store else "all")
         out(U, params={**e.params, "lane0_only": True} if store else None, sync=self.operand[e.invars[0]] in self.ordered)
 
+    def fence(self) -> JaxprEqn:
+        # (the rewrites take it for granted that an equation has a result)
+        return JaxprEqn([], [Var(ShapedArray((), "bool"))], primitive("lane_sync"), {"lanes": self.b})
+
     def lane(self, eqns: list[JaxprEqn]) -> Var:
         v = Var(ShapedArray((), "int32"))
         eqns.append(JaxprEqn([], [v], primitive("lane_index"), {"lanes": self.b}))
@@ -210,8 +214,7 @@ class _Pass:
                 nouts.append(nv)
             new = JaxprEqn(invars if invars is not None else [a(x) for x in e.invars], nouts,
                            primitive(prim or name), params if params is not None else dict(e.params))
-            fence = [JaxprEqn([], [], primitive("lane_sync"), {"lanes": self.b})] if sync else []
-            eqns.extend([*fence, new, *fence])
+            eqns.extend([self.fence(), new, self.fence()] if sync else [new])
 
         if name in _ELEMENTWISE:
             if L in ins_st:

@@ -168,15 +168,16 @@ def test_stores_of_one_element_stay_in_one_lane(name):
     assert not isinstance(plan_of(trace(call._staged, *args)), SpreadPlan)
 
 
+@pytest.mark.parametrize("mode", ["safe", "relaxed", "fast", "reproducible"])
 @pytest.mark.parametrize("name", sorted(LANE_ROWS))
-def test_lane_rows_are_synchronised_where_lanes_meet(name):
+def test_lane_rows_are_synchronised_where_lanes_meet(name, mode):
     """Lane 0's stores, and what every lane reads, stand between barriers
     (of the wavefront, where it is the whole instance)."""
     call, args = LANE_ROWS[name](np.random.default_rng(1))
     spec = trace(call._staged, *args)
     plan = plan_of(spec)
     assert isinstance(plan, LanePlan)
-    lines = emit_hip(spec, math_mode="safe").split('extern "C"')[-1].splitlines()
+    lines = emit_hip(spec, math_mode=mode).split('extern "C"')[-1].splitlines()
     sync = ("__syncthreads();",) if plan.lanes > 64 else ("__builtin_amdgcn_wave_barrier();",
                                                           '__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");')
     guards = [i for i, x in enumerate(lines) if x.lstrip().startswith("if (_lane == 0) {")]
