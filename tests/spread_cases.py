@@ -283,11 +283,18 @@ def overwritten(b, order):
     return make
 
 
-OVERWRITTEN = {f"{order}_{b if isinstance(b, int) else '%dx%d' % b}": overwritten(b, order) for order, b in
-               (("last", 100), ("last", 1000), ("first", 1000), ("loop", 1000), ("branch", 300), ("last", (8, 100)),
-                ("first", (8, 100)), ("row", (8, 100)), ("row", (300, 20)), ("column", (8, 100)), ("column", (3, 700)))}
+def _overwritten(*cases):
+    return {f"{order}_{b if isinstance(b, int) else '%dx%d' % b}": overwritten(b, order) for order, b in cases}
+
+
+# (In one lane a block lies in scratch, which every hardware queue keeps for
+# all waves of the chip: the blocks that run are small.)
+OVERWRITTEN = _overwritten(("last", 100), ("last", 300), ("first", 300), ("loop", 300), ("branch", 300), ("last", (3, 100)),
+                           ("first", (3, 100)), ("row", (3, 100)), ("row", (70, 4)), ("column", (3, 100)), ("column", (20, 16)))
+OVERWRITTEN_WIDE = _overwritten(("last", 1000), ("first", 1000), ("loop", 1000), ("branch", 3000), ("row", (8, 100)),
+                                ("row", (300, 20)), ("column", (3, 700)))
 # The rest of the block is not written: compared where it is.
-CROSSED = {f"cross_{m}x{w}": overwritten((m, w), "cross") for m, w in ((8, 100), (20, 20))}
+CROSSED = {f"cross_{m}x{w}": overwritten((m, w), "cross") for m, w in ((3, 100), (16, 20))}
 
 
 def read_by_all(b):
@@ -314,9 +321,8 @@ def read_by_all(b):
 
 
 # The same where a block's rows have a lane each.
-LANE_ROWS = {**{f"{order}_{b if isinstance(b, int) else '%dx%d' % b}": overwritten(b, order) for order, b in
-                (("last", 64), ("last", 256), ("first", 1024), ("loop", 256), ("branch", 128), ("last", (128, 4)),
-                 ("first", (128, 4)), ("row", (256, 3)), ("row", (64, 3)))},
+LANE_ROWS = {**_overwritten(("last", 64), ("last", 256), ("first", 1024), ("loop", 256), ("branch", 128), ("last", (128, 4)),
+                            ("first", (128, 4)), ("row", (256, 3)), ("row", (64, 3))),
              **{f"read_by_all_{b}": read_by_all(b) for b in (64, 256, 1024)}}
 
 

@@ -14,7 +14,7 @@ from palladium_amd.frontend import jnp, lax, pl
 from palladium_amd.frontend.core import current_builder
 from palladium_amd.ir import ShapedArray
 from palladium_amd.trace import trace
-from spread_cases import CASES, CROSSED, LANE_ROWS, MOMENTS, OVERWRITTEN
+from spread_cases import CASES, CROSSED, LANE_ROWS, MOMENTS, OVERWRITTEN, OVERWRITTEN_WIDE
 
 F = np.float32
 
@@ -161,10 +161,10 @@ def test_other_forms_keep_their_lowering(kernel):
     emit_hip(spec, math_mode="fast")
 
 
-@pytest.mark.parametrize("name", sorted({**OVERWRITTEN, **CROSSED}))
+@pytest.mark.parametrize("name", sorted({**OVERWRITTEN, **OVERWRITTEN_WIDE, **CROSSED}))
 def test_stores_of_one_element_stay_in_one_lane(name):
     """Lanes are not ordered: an element that two stores write has one lane."""
-    call, args = {**OVERWRITTEN, **CROSSED}[name](np.random.default_rng(1))
+    call, args = {**OVERWRITTEN, **OVERWRITTEN_WIDE, **CROSSED}[name](np.random.default_rng(1))
     assert not isinstance(plan_of(trace(call._staged, *args)), SpreadPlan)
 
 
