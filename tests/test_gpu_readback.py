@@ -58,3 +58,26 @@ def test_packed_inputs_of_mixed_types(n):
     pending = [f.launch(*c) for c in calls]  # more than the sets in flight
     for p, (a, b, c) in zip(pending, calls):
         np.testing.assert_array_equal(p.wait(), a + b.astype(np.float32) * np.where(c, np.float32(2), np.float32(1)))
+
+
+@pytest.mark.parametrize("shapes", [((5,), (0,), (5,)), ((0,), (5,), (5,)), ((5,), (5,), (0,))])
+def test_packed_inputs_with_an_empty_one(shapes):
+    """An input without elements takes no place among the packed ones."""
+    full = [k for k, s in enumerate(shapes) if s != (0,)]
+
+    def kernel(*refs):
+        refs[-1][...] = refs[full[0]][...] - refs[full[1]][...]
+
+    specs = [pl.BlockSpec((1,), lambda i: (i,)) if s != (0,) else pl.BlockSpec((0,), lambda i: (0,)) for s in shapes]
+    f = pa.hip_call(kernel, grid=(5,), in_specs=specs, out_specs=pl.BlockSpec((1,), lambda i: (i,)),
+                    out_shape=pl.ShapeDtypeStruct((5,), np.float32), math_mode="safe")
+    args = [np.random.default_rng(k).standard_normal(s).astype(np.float32) for k, s in enumerate(shapes)]
+    np.testing.assert_array_equal(f(*args), args[full[0]] - args[full[1]])
+
+
+def test_nothing_but_empty_inputs():
+    def kernel(e_ref, o_ref):
+        o_ref[...] = jnp.full((3,), 2.0, jnp.float32)
+
+    f = pa.hip_call(kernel, out_shape=pl.ShapeDtypeStruct((3,), np.float32), math_mode="safe")
+    np.testing.assert_array_equal(f(np.zeros(0, np.float32)), np.full(3, 2, np.float32))
