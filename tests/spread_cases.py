@@ -332,7 +332,7 @@ def moments(m, w, n, dt="f32"):
         x = x_ref[...]
         z = x
         for _ in range(n):
-            z = x - jnp.sum(z, axis=1, keepdims=True) * 0.125
+            z = x - jnp.sum(z, axis=1, keepdims=True) * (0.5 / w)
         o_ref[...] = z
         n_ref[...] = jnp.sum(jnp.where(z > x, 0.5, 0.25), axis=1)
 
