@@ -69,6 +69,7 @@ def _operand(expr: str, src_ctype: str) -> str:
 
 def _tmpl(opname: str, ops: list[CVal], out_ctype: str) -> str:
     f = _is_float(ops[0]) if ops else False
+    minus = "({a})" if ops and ops[0].expr.startswith("-") else "{a}"  # of a negative literal: no --
     if opname == "add":
         return "({a} + {b})"
     if opname == "sub":
@@ -96,7 +97,7 @@ def _tmpl(opname: str, ops: list[CVal], out_ctype: str) -> str:
     if opname == "pow_with_log":
         return "ph_pow_with_log({a}, {b}, {c})"
     if opname == "neg":
-        return "(-{a})"
+        return f"(-{minus})"
     if opname == "abs":
         if f:
             return "fabsf({a})"
@@ -119,7 +120,7 @@ def _tmpl(opname: str, ops: list[CVal], out_ctype: str) -> str:
         "floor": "floorf({a})",
         "ceil": "ceilf({a})",
         "round": "roundf({a})",
-        "logistic": "(1.0f / (1.0f + ph_exp(-{a})))",
+        "logistic": f"(1.0f / (1.0f + ph_exp(-{minus})))",
         "atan2": "atan2f({a}, {b})",
     }
     if opname in unary_f:

@@ -298,3 +298,16 @@ def test_views_step_over_what_they_leave_out(shape, index):
         at = view.at(str(i))
         assert at.startswith(name + "[") and base + eval(at[len(name) + 1:-1].replace("/", "//")) == w
     assert (view.steps is None) == bool((np.diff(want) == 1).all())
+
+
+@pytest.mark.parametrize("shape, grid", [((1,), 64), ((40,), 5), ((64, 3), 2)])
+def test_negatives_of_negative_constants_compile(shape, grid):
+    """In a scalar, in a block over lanes and in rows over lanes, where a
+    constant stands for itself."""
+    def k(x_ref, o_ref):
+        c = jnp.full(shape, -0.75, jnp.float32)
+        o_ref[...] = x_ref[...] * -c + jnp.logistic(c)
+
+    s = pl.BlockSpec(shape, lambda i: (i,) + (0,) * (len(shape) - 1))
+    full = (grid * shape[0], *shape[1:])
+    _compile(_spec(k, pl.ShapeDtypeStruct(full, F), np.zeros(full, F), grid=(grid,), in_specs=[s], out_specs=s))
