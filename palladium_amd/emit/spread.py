@@ -25,6 +25,11 @@ A product of whole input blocks, (M, K) @ (K, W), is computed in 16 x 16
 tiles by the matrix cores (`_tile_plan`): the block's elements then lie in
 lanes as those leave them, and what follows is element-wise on that.
 
+Nothing orders the lanes of an instance, which may lie in several workgroups.
+So an element has one lane: a kernel of which two stores may meet in an
+element from different lanes, or that reads an output where another lane wrote
+it, is not taken.
+
 Control flow is uniform within an instance, as in `lanes`: a loop condition
 or switch index that varies along the block is not taken, neither is
 anything else outside these forms (`spread_transform` returns None and the
@@ -77,8 +82,9 @@ FEW_INSTANCES = 16_384
 # A call without a grid is documented as one instance on one lane, and
 # `explain` names the fix (a grid and BlockSpecs): it keeps that form unless
 # it loops over more elements than one lane can hold unrolled, or multiplies
-# matrices. (A grid of one instance is spread: 1,000 float32 values in one block
-# took 147 us in one lane, 5.4 over lanes.)
+# matrices. The form is kept for what it says, not for its time: a grid of one
+# instance is spread, and 1,000 float32 values in one block took 147 us in one
+# lane and take 5.4 over lanes (on the device; either call adds the launch).
 MIN_SINGLE = 65
 # A lane-parallel kernel (block rows across lanes) whose rows are this long
 # is spread along the rows instead, so a wavefront reads whole lines and not
@@ -91,7 +97,8 @@ MIN_ROW = 8
 # regroup bfloat16 arithmetic across operations: x * y + c * x becomes
 # x * (y + c), the sum rounded to 16 bits. One lane that held this many values
 # had them in memory, every operation rounded as the interpreter does, and
-# blocks of them still round so (`ROUNDED_PRELUDE`). Shorter ones were in
+# blocks of them still round so (`ROUNDED_PRELUDE`), after a product in tiles
+# too. Shorter ones were in
 # registers then too, as are the rows of a lane-parallel kernel. Results of
 # x * y + 0.1 x - y / (x^2 + 1) that differ from the one-lane form's, rounded /
 # regrouped: 28.9 / 0 % of them in blocks of 16, 18.5 / 7.6 of 24, 11.6 / 15.5
@@ -1295,9 +1302,10 @@ def _rule_spread_dot(env: Environment, cursor: Cursor, eqn: JaxprEqn) -> None:
     for its own elements (4 rows a tile, one column), four k at a time.
 
     Rows x (64, 32) + bias, tanh, 262,144 rows: float32 280 -> 22 us (4.6
-    TB/s of the 101 MB it cannot do without, HBM the bound), bfloat16 257 ->
-    12.7, in order 547 -> 46; (128, 64) bfloat16 1,162 -> 28 us. A row per
-    lane read its row from memory once per column."""
+    TB/s of the 101 MB it cannot do without), bfloat16 257 -> 12.7, in order
+    547 -> 46; (128, 64) bfloat16 1,162 -> 28 us. A row per lane read its row
+    from memory once per column. What is left is the way through the caches: a
+    wavefront of 32 rows (8 KB there) loads all the weights (8 KB) again."""
     plan = env.spread  # type: ignore[attr-defined]
     mode = getattr(env, "math_mode", None)
     lhs, rhs = env.val(eqn.invars[0]), env.val(eqn.invars[1])
