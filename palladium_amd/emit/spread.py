@@ -1259,13 +1259,14 @@ def _ordered_sum(env: Environment, cursor: Cursor, plan: SpreadPlan, src: CVal, 
     """init 0, then one add per element in index order, in the type a lane
     alone accumulates in (bfloat16 sums in float32, rounded once)."""
     act = "float" if ct == "__bf16" else ct
-    stride = row_stride(plan.width)
+    # the same bytes a row in every type: teams of other wavefronts may be a sum ahead
+    stride = row_stride(plan.width) * (2 if act == "_Float16" else 1)
     teams = max(1, env.spread_block // plan.team)  # type: ignore[attr-defined]
     row, acc = cursor.fresh("_rp"), cursor.fresh("_acc")
     sync = "__syncthreads();" if plan.team > WAVE else "ph_wave_sync();"
     # One array for all sums of a kernel (each ends with its reads done): the
     # compiler adds up those of a kernel, and three of 58 KB are past the CU's.
-    env.staged = max(getattr(env, "staged", 0), teams * stride * (2 if act == "_Float16" else 4))  # type: ignore[attr-defined]
+    env.staged = teams * row_stride(plan.width) * 4  # type: ignore[attr-defined]
     at = f"(threadIdx.x / {plan.team}u) * {stride}u" if teams > 1 else "0"
     cursor.emit(f"{act}* {row} = ({act}*){STAGING} + {at};")
     for s in range(plan.slots):

@@ -2,6 +2,8 @@
 form, that its lanes cover every element once, and the forms it leaves to
 the other lowerings. (The results are compared on the GPU.)"""
 
+import re
+
 import numpy as np
 import pytest
 
@@ -107,6 +109,25 @@ def test_large_grids_stay_below_the_lane_limit(kind, m, w):
         if grid == edge:
             assert isinstance(plan, SpreadPlan)
         emit_hip(spec, math_mode="fast")
+
+
+@pytest.mark.parametrize("name", sorted(n for n in {**CASES, **MOMENTS} if n.startswith(("rows", "moments"))))
+def test_a_team_stages_every_sum_in_its_own_bytes(name):
+    """A wavefront may be a sum ahead of the others, in another type."""
+    call, args = {**CASES, **MOMENTS}[name](np.random.default_rng(1))
+    text = emit_hip(trace(call._staged, *args), math_mode="safe")
+    rows = re.findall(r"\((\w+)\*\)_rows \+ \(threadIdx.x / (\d+)u\) \* (\d+)u;", text)
+    alone = re.findall(r"\(\w+\*\)_rows \+ 0;", text)
+    total = re.search(r"_rows\[(\d+)\];", text)
+    if not rows and not alone:
+        assert total is None
+        return
+    assert not (rows and alone)
+    places = {(int(team), int(pitch) * (2 if t == "_Float16" else 4)) for t, team, pitch in rows}
+    assert len(places) <= 1
+    for team, pitch in places:
+        plan = plan_of(trace(call._staged, *args))
+        assert pitch >= 4 * plan.width and pitch * (launch_geometry(trace(call._staged, *args)).block // team) <= int(total[1])
 
 
 @pytest.mark.parametrize("name, rounds", [("flat_250_bf16", True), ("flat_1250_bf16", True), ("flat_wide_bf16", True),
